@@ -2108,6 +2108,7 @@ int level_autotune(Level *L) {
                 // primitives, norms): it is timed with the residual, reading B
                 // and writing C so that the state in A stays as it was
                 ResArgs rp = r;
+                rp.partials = L->partials;  // rebuild_tiles grows (frees) it with the tile count
                 rp.st.src = L->view[1];
                 rp.dst = L->view[2];
                 rp.do_chem = c->prm.do_chemistry;

@@ -119,3 +119,24 @@ def test_porous_tiny_boxes():
     assert len(c.boxes) > 100
     _check(c, 3, mode=abi.MODE_BATCHED)
     _check(c, 2, mode=abi.MODE_PER_BOX)
+
+
+def test_autotune_when_a_candidate_has_more_tiles():
+    """64 boxes of 16x16x2: 8 cell tiles a box with the default shape 64,2,2 and
+    16 with the candidate 64,1,4, so the buffer of the tiles' partial sums grows
+    between two candidates; the post-step pass then writes the new buffer"""
+    from mesoflow_amd import runtime
+    c = cases.porous_reactor(n_cell=(32, 32, 32), nspec=5, nreact=2, geometry="spheres", porosity=0.6, rmin=3, rmax=5,
+                             order_hyp=5, seed=13, max_grid_size=(16, 16, 2))
+    s0 = c.make_state()
+    want, winfo = run_gpu(c, 3, state=s0)
+    ctx = runtime.Context(c)
+    L = runtime.Level(ctx)
+    L.set_state(s0)
+    L.autotune()
+    L.step(3)
+    got, ginfo = L.get_state(), L.info()
+    L.close()
+    ctx.close()
+    assert np.array_equal(got, want)
+    assert ginfo[:3] == winfo[:3]
