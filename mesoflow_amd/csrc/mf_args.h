@@ -196,7 +196,7 @@ struct BoxPostArgs {
 struct KernelSet {
     int ns;
     bool has_bg_gas;           // the family's thermo has a background gas (using_bg_inertgas)
-    void (*fill)(const FillArgs &, int phase, hipStream_t);
+    void (*fill)(const FillArgs &, hipStream_t);
     // physical-boundary phase of the fill over the region [rlo, rhi] of a.s
     void (*fill_region)(const FillArgs &, int phase, const int *rlo, const int *rhi, hipStream_t);
     // physical-boundary phase of the fill over a list of cells ([3][n])

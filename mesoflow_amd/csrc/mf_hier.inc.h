@@ -649,7 +649,7 @@ void hier_fill_fine(Hier *H, double *dst, double *c_old, double *c_new, int stag
     FillArgs fa = fill_args(Lc, H->ct, stage);
     if (mode_forced >= 0) { fa.ts = nullptr; fa.time_host = time_host; }
     else fa.ts = Lf->ts;
-    for (int ph = 0; ph <= 3; ++ph) c->ks->fill(fa, ph, st);
+    c->ks->fill(fa, st);
     const View fv = padded_view(dst, Lf->n, nv);
     if (nfcf)
         hipLaunchKernelGGL(k_hier_cf, dim3(hgrid((int64_t)nfcf * nv)), dim3(256), 0, st, fv, ctv, fcf, fcfm, nfcf, nv,
@@ -674,7 +674,7 @@ void hier_stage(Hier *H, int lev, int stage, int mode, double *c_old, double *c_
     const double w = stage == 3 ? kTwo3rd : kTwo3rd * kHalf * kHalf;
     if (lev == 0) {
         FillArgs f = fill_args(L, src, stage);
-        for (int ph = 0; ph <= 3; ++ph) c->ks->fill(f, ph, st);
+        c->ks->fill(f, st);
     } else {
         hier_fill_fine(H, src, c_old, c_new, stage, -1, 0.0, H->cneed, H->ncneed, H->fcf, H->fcfm, H->nfcf, true);
     }

@@ -271,11 +271,7 @@ MFD void face_flux(const Tab &T, const Acc &acc, const StageArgs &a, int i, int 
                     } else if (c == RHOE) fc[q] = (uc[q] + pr[q][4]) * vn;
                     else fc[q] = uc[q] * vn;
                 }
-                double fp = N::weno_plus(fc[0], fc[1], fc[2], fc[3], fc[4]);
-                double fm = N::weno_minus(fc[1], fc[2], fc[3], fc[4], fc[5]);
-                double up = N::weno_plus(uc[0], uc[1], uc[2], uc[3], uc[4]);
-                double um = N::weno_minus(uc[1], uc[2], uc[3], uc[4], uc[5]);
-                fput(c, adv(c, kHalf * (fp + lam * up) + kHalf * (fm - lam * um)));
+                fput(c, adv(c, N::weno_llf(uc, fc, lam)));
             }
         } else if (ORDER == 1 || ORDER == 2) {
             double ul[NC], ur[NC], fh[NC];
@@ -414,7 +410,7 @@ struct LdsCell {
     MFD double operator()(int n) const {
         if (n < NCV) return rec[n];
         if (n >= FLO) return rec[NCV + n - FLO];
-        if (n == VFRAC) return rec[NC + 5];
+        if (n == VFRAC) return rec[NC + 3];
         return sel_get(*acc, i, j, k, n, cid);
     }
 };
@@ -438,6 +434,10 @@ MFD double pick(const double (&v)[M], int s) {
     for (int q = 0; q < M; ++q) r = (q == s) ? v[q] : r;
     return r;
 }
+// doubles of a staged cell: the flux components' states, the normal velocity,
+// pressure, gamma and vfrac
+template <class P>
+constexpr int kFaceRec = (Num<P>::NC + 4) | 1;
 template <class P, int D>
 __global__ __launch_bounds__(512, MF_FACE_MIN_WAVES) void k_faces_lds(StageArgs a, Work w) {
     using N = Num<P>;
@@ -446,7 +446,7 @@ __global__ __launch_bounds__(512, MF_FACE_MIN_WAVES) void k_faces_lds(StageArgs 
     constexpr int T1 = (D + 1) % 3, T2 = (D + 2) % 3;
     // LDS tile: one record of FS doubles per stencil cell (an odd stride keeps
     // 64-bit reads of consecutive cells on distinct banks)
-    constexpr int FVX = NC, FP = NC + 3, FG = NC + 4, FVF = NC + 5, NF = NC + 6, FS = NF | 1;
+    constexpr int FVN = NC, FP = NC + 1, FG = NC + 2, FVF = NC + 3, FS = kFaceRec<P>;
     static_assert(P::kGammaIgnoresP, "the staged gamma needs a gamma that does not depend on the pressure");
     extern __shared__ double lds[];
     if (step_skipped(a.ts)) return;
@@ -485,9 +485,7 @@ __global__ __launch_bounds__(512, MF_FACE_MIN_WAVES) void k_faces_lds(StageArgs 
             for (int c = 0; c < NC; ++c) rec[c] = u[c];
             double vx, vy, vz, p;
             N::euler_prims(T, u, vx, vy, vz, p);
-            rec[FVX + 0] = vx;
-            rec[FVX + 1] = vy;
-            rec[FVX + 2] = vz;
+            rec[FVN] = D == 0 ? vx : (D == 1 ? vy : vz);
             rec[FP] = p;
             rec[FG] = P::get_gama_from_rpc(T, u[RHO], p, u + NCV);
             rec[FVF] = cp(VFRAC);
@@ -547,7 +545,7 @@ __global__ __launch_bounds__(512, MF_FACE_MIN_WAVES) void k_faces_lds(StageArgs 
                     double rhoeR = ur[RHOE] - kHalf * (ur[RHOU] * ur[RHOU] + ur[RHOV] * ur[RHOV] + ur[RHOW] * ur[RHOW]) / ur[RHO];
                     double presL = P::get_p_from_rec(T, rhoeL, ul[RHO], ul + NCV);
                     double presR = P::get_p_from_rec(T, rhoeR, ur[RHO], ul + NCV);
-                    double veln = std_max(fabs(recL[FVX + D]), fabs(recR[FVX + D]));
+                    double veln = std_max(fabs(recL[FVN]), fabs(recR[FVN]));
                     double gamaL = recL[FG], gamaR = recR[FG];
                     double ahalf = std_max(sqrt(gamaL * presL / ul[RHO]), sqrt(gamaR * presR / ur[RHO]));
                     lam = ahalf + veln;
@@ -578,21 +576,13 @@ __global__ __launch_bounds__(512, MF_FACE_MIN_WAVES) void k_faces_lds(StageArgs 
                     for (int q = 0; q < 6; ++q) {
                         const double *rq = rs[q];
                         uc[q] = rq[c];
-                        const double vn = rq[FVX + D];
-                        if (c == RHO) fc[q] = uc[q] * vn;
-                        else if (c >= RHOU && c <= RHOW) {
-                            const double va = rq[FVX + (c - RHOU)];
-                            const double mm = rq[RHO] * va;
-                            fc[q] = (c - RHOU == D) ? (mm * va + rq[FP]) : (mm * vn);
-                        } else if (c == RHOE) fc[q] = (uc[q] + rq[FP]) * vn;
+                        const double vn = rq[FVN];
+                        // geteulerflux with rho v_a taken as the momentum itself
+                        if (c == RHOU + D) fc[q] = fma(uc[q], vn, rq[FP]);
+                        else if (c == RHOE) fc[q] = (uc[q] + rq[FP]) * vn;
                         else fc[q] = uc[q] * vn;
                     }
-                    double fp = N::weno_plus(fc[0], fc[1], fc[2], fc[3], fc[4]);
-                    double fm = N::weno_minus(fc[1], fc[2], fc[3], fc[4], fc[5]);
-                    double up = N::weno_plus(uc[0], uc[1], uc[2], uc[3], uc[4]);
-                    double um = N::weno_minus(uc[1], uc[2], uc[3], uc[4], uc[5]);
-                    const double h = kHalf * (fp + lam * up) + kHalf * (fm - lam * um);
-                    hc[c] = c < NCV ? h : T.advect_flag[c - NCV] * h;
+                    hc[c] = N::weno_llf(uc, fc, lam);
                 }
             }
             // ---- viscous stress and work (:293-367), conduction (:373-374), species diffusion (:425-428)
@@ -690,21 +680,9 @@ __global__ __launch_bounds__(512, MF_FACE_MIN_WAVES) void k_faces_lds(StageArgs 
                     for (int q = 0; q < 6; ++q) {
                         const double *rq = rs[q];
                         uc[q] = rq[c];
-                        const double vn = rq[FVX + D];
-                        if (c == RHO) fc[q] = uc[q] * vn;
-                        else if (c >= RHOU && c <= RHOW) {
-                            const double va = rq[FVX + (c - RHOU)];
-                            const double mm = rq[RHO] * va;
-                            fc[q] = (c - RHOU == D) ? (mm * va + rq[FP]) : (mm * vn);
-                        } else if (c == RHOE) fc[q] = (uc[q] + rq[FP]) * vn;
-                        else fc[q] = uc[q] * vn;
+                        fc[q] = uc[q] * rq[FVN];
                     }
-                    double fp = N::weno_plus(fc[0], fc[1], fc[2], fc[3], fc[4]);
-                    double fm = N::weno_minus(fc[1], fc[2], fc[3], fc[4], fc[5]);
-                    double up = N::weno_plus(uc[0], uc[1], uc[2], uc[3], uc[4]);
-                    double um = N::weno_minus(uc[1], uc[2], uc[3], uc[4], uc[5]);
-                    const double h = kHalf * (fp + lam * up) + kHalf * (fm - lam * um);
-                    hc[c] = c < NCV ? h : T.advect_flag[c - NCV] * h;
+                    hc[c] = T.advect_flag[c - NCV] * N::weno_llf(uc, fc, lam);
                 }
             }
 #pragma unroll
@@ -742,6 +720,10 @@ MFD void chemistry_rk3(const Tab &T, double *S, double dt) {
     double S0[NS], F[3][NS], st[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) S0[s] = S[FLO + s];
+    // the temperature does not change over the stages: the rate constants once,
+    // where each stage's source would evaluate the same exponentials
+    double rates[MF_MAX_REACTIONS];
+    P::rate_constants(T, S[TEMP], rates);
     const double a10 = 1.0, a20 = 0.25, a21 = 0.25;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -753,7 +735,7 @@ MFD void chemistry_rk3(const Tab &T, double *S, double dt) {
             st[s] = v;
         }
         double src[NS];
-        P::spec_source(T, ChemCell<NS>{S, st}, src);
+        P::spec_source_k(T, rates, ChemCell<NS>{S, st}, src);
 #pragma unroll
         for (int s = 0; s < NS; ++s) F[k][s] = 0.0 + src[s];
     }
@@ -1215,6 +1197,31 @@ MFD void fill_cell_rules(const FillArgs &a, const int *iv, int phase, const Tab 
     }
 }
 
+// ghost cell q of a padded level array: the z slabs, then the y slabs of the
+// valid z planes, then the x slabs of the valid rows
+MFD void ghost_cell(int64_t q, int64_t nzs, int64_t nys, int PX, int PY, int nx, int ny, int nz, int *iv) {
+    const int G = MF_NGROW;
+    if (q < nzs) {
+        int64_t r = q;
+        iv[0] = (int)(r % PX) - G; r /= PX;
+        iv[1] = (int)(r % PY) - G; r /= PY;
+        int g = (int)r;
+        iv[2] = g < G ? g - G : nz + (g - G);
+    } else if (q < nzs + nys) {
+        int64_t r = q - nzs;
+        iv[0] = (int)(r % PX) - G; r /= PX;
+        int g = (int)(r % (2 * G)); r /= (2 * G);
+        iv[1] = g < G ? g - G : ny + (g - G);
+        iv[2] = (int)r;
+    } else {
+        int64_t r = q - nzs - nys;
+        int g = (int)(r % (2 * G)); r /= (2 * G);
+        iv[0] = g < G ? g - G : nx + (g - G);
+        iv[1] = (int)(r % ny); r /= ny;
+        iv[2] = (int)r;
+    }
+}
+
 template <class P>
 __global__ __launch_bounds__(256) void k_fill(FillArgs a, int phase) {
     if (step_skipped(a.ts)) return;
@@ -1229,26 +1236,96 @@ __global__ __launch_bounds__(256) void k_fill(FillArgs a, int phase) {
     const int64_t total = nzs + nys + nxs;
     for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
         int iv[3];
-        if (q < nzs) {
-            int64_t r = q;
-            iv[0] = (int)(r % PX) - G; r /= PX;
-            iv[1] = (int)(r % PY) - G; r /= PY;
-            int g = (int)r;
-            iv[2] = g < G ? g - G : nz + (g - G);
-        } else if (q < nzs + nys) {
-            int64_t r = q - nzs;
-            iv[0] = (int)(r % PX) - G; r /= PX;
-            int g = (int)(r % (2 * G)); r /= (2 * G);
-            iv[1] = g < G ? g - G : ny + (g - G);
-            iv[2] = (int)r;
-        } else {
-            int64_t r = q - nzs - nys;
-            int g = (int)(r % (2 * G)); r /= (2 * G);
-            iv[0] = g < G ? g - G : nx + (g - G);
-            iv[1] = (int)(r % ny); r /= ny;
-            iv[2] = (int)r;
-        }
+        ghost_cell(q, nzs, nys, PX, PY, nx, ny, nz, iv);
         fill_cell_rules<P>(a, iv, phase, T, time);
+    }
+}
+
+// All phases of k_fill in one launch. The rule that decides a ghost cell (the
+// last ext_dir direction it lies outside of, else the last foextrap or wall
+// one) reads a cell with one outside direction fewer, so every ghost cell is a
+// chain of at most three rules over one valid cell: the chain is walked to that
+// cell and its rules are applied on the way back, with the arithmetic of the
+// phases. It reads valid cells only (no order between ghost cells) and needs
+// every rule's source one step inside: at least MF_NGROW cells per direction.
+// Bound by launches at small sizes: four dependent launches a stage became one
+// (19 -> 6 us a stage for 32x4x4 cells).
+template <class P>
+__global__ __launch_bounds__(256) void k_fill_all(FillArgs a) {
+    constexpr int NV = Num<P>::NV;
+    if (step_skipped(a.ts)) return;
+    const Tab &T = *a.tab;
+    const double time = !a.ts ? a.time_host : (a.stage == 1 ? a.ts->t : a.ts->t + a.ts->dt);
+    const int G = MF_NGROW;
+    const int nx = a.n[0], ny = a.n[1], nz = a.n[2];
+    const int PX = nx + 2 * G, PY = ny + 2 * G;
+    const int64_t nzs = (int64_t)2 * G * PX * PY;
+    const int64_t nys = (int64_t)nz * 2 * G * PX;
+    const int64_t nxs = (int64_t)nz * ny * 2 * G;
+    const int64_t total = nzs + nys + nxs;
+    for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
+        int iv[3];
+        ghost_cell(q, nzs, nys, PX, PY, nx, ny, nz, iv);
+        // the chain: the direction of each rule and the position it applies at
+        int at[3][3], dir[3], nr = 0, c[3] = {iv[0], iv[1], iv[2]};
+#pragma unroll
+        for (int step = 0; step < 3; ++step) {
+            int pick = -1;
+            bool ext = false;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                if (a.periodic[d] || (c[d] >= 0 && c[d] < a.n[d])) continue;
+                const bool e = (c[d] < 0 ? a.lo_bc[d] : a.hi_bc[d]) == MF_BC_EXT_DIR;
+                if (e || !ext) { pick = d; ext = e; }
+            }
+            if (pick < 0) break;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) at[step][d] = c[d];
+            dir[step] = pick;
+            nr = step + 1;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                if (d != pick) continue;
+                const bool low = c[d] < 0;
+                const int bc = low ? a.lo_bc[d] : a.hi_bc[d];
+                if (bc == MF_BC_WALL) c[d] = low ? -c[d] - 1 : 2 * (a.n[d] - 1) - c[d] + 1;
+                else c[d] = low ? 0 : a.n[d] - 1;
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (c[d] < 0) c[d] += a.n[d];
+            else if (c[d] >= a.n[d]) c[d] -= a.n[d];
+        }
+        double v[NV];
+        const double *src = a.s.p + a.s.off(c[0], c[1], c[2]);
+#pragma unroll
+        for (int n = 0; n < NV; ++n) v[n] = src[(int64_t)n * a.s.ns];
+#pragma unroll
+        for (int step = 2; step >= 0; --step) {
+            if (step >= nr) continue;
+            const int d = dir[step];
+            const int pd = d == 0 ? at[step][0] : (d == 1 ? at[step][1] : at[step][2]);
+            const bool low = pd < 0;
+            const int bc = low ? a.lo_bc[d] : a.hi_bc[d];
+            if (bc == MF_BC_EXT_DIR) {
+                double x[3], e[NV];
+#pragma unroll
+                for (int m = 0; m < 3; ++m) x[m] = a.prob_lo[m] + (at[step][m] + 0.5) * a.dx[m];
+#pragma unroll
+                for (int n = 0; n < NV; ++n) e[n] = 0.0;
+                P::externalbc(T, x, v, e, d, low ? 1 : -1, time);
+#pragma unroll
+                for (int n = 0; n < NV; ++n) v[n] = e[n];
+            } else if (bc == MF_BC_WALL) {
+#pragma unroll
+                for (int n = 0; n < NV; ++n)
+                    if (n == RHOU || n == RHOV || n == RHOW || n == VELX || n == VELY || n == VELZ) v[n] = -v[n];
+            }
+        }
+        double *dst = a.s.p + a.s.off(iv[0], iv[1], iv[2]);
+#pragma unroll
+        for (int n = 0; n < NV; ++n) dst[(int64_t)n * a.s.ns] = v[n];
     }
 }
 
@@ -1505,82 +1582,88 @@ __global__ __launch_bounds__(128) void k_cut_geom_sub(CutArgs a, double *geom, u
     for (int w = 0; w < 4; ++w) mask[(int64_t)w * a.ncut + q] = mb[w];
 }
 
-// update_cutcells of the level's cut-cell list (ib_utils.H:271-436), one thread
-// per cut cell, with the static geometry of k_cut_geom: the IDW sums run over
-// the fluid neighbours of the mask in the reference's loop order.
+// The IDW sums of one cut cell over its fluid neighbours, by 8 lanes: a lane
+// takes the rows r = lane, lane + 8, .. of the 25 rows (m, n) of five cells, so
+// that neighbours next to each other in memory are read one after the other
+// and a cell's 125 positions are 20 steps long instead of 125; the lanes' sums
+// are then exchanged. One thread a cell walked its neighbours serially: 84 us
+// for the 35 thousand cut cells of a 64^3 reactor, whatever their number.
+template <int NS>
+struct CutSums {
+    double su0, su1, su2, swv, sp, sT, sR, swn, sS[NS];
+};
+template <int NS>
+MFD void cut_row(const CutArgs &a, const double *c0, int m, int n, unsigned bits, const double *dnd, const double *xnd,
+                 bool vel0, CutSums<NS> &o) {
+    const int64_t ns = a.s.ns;
+    const bool doT = !a.conj_ht, doS = !a.spec_in_solid;
+    const double a1 = m * dnd[1], a2 = n * dnd[2], y1 = a1 - xnd[1], y2 = a2 - xnd[2];
+    while (bits) {
+        const int l = __ffs(bits) - 3;
+        bits &= bits - 1;
+        const double *c = c0 + l;
+        const double a0 = l * dnd[0], y0 = a0 - xnd[0];
+        // one reciprocal per weight, multiplied into each value (the
+        // reference divides every value by the squared distance)
+        if (!vel0 && !(l == 0 && m == 0 && n == 0)) {
+            const double iw = div_pos(1.0, a0 * a0 + a1 * a1 + a2 * a2 + kTiny2);
+            o.su0 += c[(int64_t)VELX * ns] * iw;
+            o.su1 += c[(int64_t)VELY * ns] * iw;
+            o.su2 += c[(int64_t)VELZ * ns] * iw;
+            o.swv += iw;
+        }
+        const double iw = div_pos(1.0, y0 * y0 + y1 * y1 + y2 * y2 + kTiny2);
+        o.sp += c[(int64_t)PRES * ns] * iw;
+        if (doT) o.sT += c[(int64_t)TEMP * ns] * iw;
+        o.sR += c[(int64_t)DENS * ns] * iw;
+        if (doS) {
+#pragma unroll
+            for (int q = 0; q < NS; ++q) o.sS[q] += c[(int64_t)(FLO + q) * ns] * iw;
+        }
+        o.swn += iw;
+    }
+}
+constexpr int kCutLanes = 8;
+template <int NS>
+__device__ __forceinline__ void cut_exchange(CutSums<NS> &o) {
+    auto red = [](double &v) {
+#pragma unroll
+        for (int d = 1; d < kCutLanes; d <<= 1) v += __shfl_xor(v, d, 64);
+    };
+    red(o.su0); red(o.su1); red(o.su2); red(o.swv);
+    red(o.sp); red(o.sT); red(o.sR); red(o.swn);
+#pragma unroll
+    for (int q = 0; q < NS; ++q) red(o.sS[q]);
+}
+// the updated components of cut cell (i, j, k) from its sums
 template <class P>
-__global__ __launch_bounds__(128) void k_cutcells(CutArgs a) {
+MFD void cut_finish(const Tab &T, const CutArgs &a, int i, int j, int k, double dist, bool vel0, const CutSums<P::NS> &o,
+                    double *out) {
     using N = Num<P>;
     constexpr int NS = P::NS, NV = N::NV;
-    if (step_skipped(a.ts)) return;
-    const int q = xcd_chunk(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (q >= a.ncut) return;
-    const Tab &T = *a.tab;
     const View &s = a.s;
-    const int i = a.list[q], j = a.list[a.ncut + q], k = a.list[2 * a.ncut + q];
-    double out[NV];
+    const bool doT = !a.conj_ht, doS = !a.spec_in_solid;
+    const double dxmin = fmin(a.dx[0], fmin(a.dx[1], a.dx[2]));
 #pragma unroll
     for (int n = 0; n < NV; ++n) out[n] = s(i, j, k, n);
-    const double *dx = a.dx;
-    const double dxmin = fmin(dx[0], fmin(dx[1], dx[2]));
-    const double dnd[3] = {dx[0] / dxmin, dx[1] / dxmin, dx[2] / dxmin};
-    const double xnd[3] = {a.geom[q], a.geom[(int64_t)a.ncut + q], a.geom[(int64_t)2 * a.ncut + q]};
-    const double dist = a.geom[(int64_t)3 * a.ncut + q];
-    const double cutoff = dxmin * 1e-5;
-    const bool doT = !a.conj_ht, doS = !a.spec_in_solid;
-    const bool vel0 = fabs(dist) < cutoff;
-    double su0 = 0.0, su1 = 0.0, su2 = 0.0, swv = 0.0;
-    double sp = 0.0, sT = 0.0, sR = 0.0, swn = 0.0, sS[NS];
-#pragma unroll
-    for (int q2 = 0; q2 < NS; ++q2) sS[q2] = 0.0;
-    for (int w = 0; w < 4; ++w) {
-        unsigned bits = a.mask[(int64_t)w * a.ncut + q];
-        while (bits) {
-            const int nb = w * 32 + __ffs(bits) - 1;
-            bits &= bits - 1;
-            const int l = nb % 5 - 2, m = (nb / 5) % 5 - 2, n = nb / 25 - 2;
-            const double *c = s.p + s.off(i + l, j + m, k + n);
-            const int64_t ns = s.ns;
-            // one reciprocal per weight, multiplied into each value (the
-            // reference divides every value by the squared distance)
-            if (!vel0 && !(l == 0 && m == 0 && n == 0)) {
-                double a0 = l * dnd[0], a1 = m * dnd[1], a2 = n * dnd[2];
-                const double iw = div_pos(1.0, a0 * a0 + a1 * a1 + a2 * a2 + kTiny2);
-                su0 += c[(int64_t)VELX * ns] * iw;
-                su1 += c[(int64_t)VELY * ns] * iw;
-                su2 += c[(int64_t)VELZ * ns] * iw;
-                swv += iw;
-            }
-            double a0 = l * dnd[0] - xnd[0], a1 = m * dnd[1] - xnd[1], a2 = n * dnd[2] - xnd[2];
-            const double iw = div_pos(1.0, a0 * a0 + a1 * a1 + a2 * a2 + kTiny2);
-            sp += c[(int64_t)PRES * ns] * iw;
-            if (doT) sT += c[(int64_t)TEMP * ns] * iw;
-            sR += c[(int64_t)DENS * ns] * iw;
-            if (doS) {
-#pragma unroll
-                for (int q2 = 0; q2 < NS; ++q2) sS[q2] += c[(int64_t)(FLO + q2) * ns] * iw;
-            }
-            swn += iw;
-        }
-    }
     // Dirichlet (u = 0) IDW of the velocities, :98-152
     if (vel0) {
         out[VELX] = 0.0; out[VELY] = 0.0; out[VELZ] = 0.0;
     } else {
         double dn = fabs(dist) / dxmin;
         double wd = 1.0 / (dn * dn);
-        out[VELX] = (su0 + 0.0 / (dn * dn)) / (swv + wd);
-        out[VELY] = (su1 + 0.0 / (dn * dn)) / (swv + wd);
-        out[VELZ] = (su2 + 0.0 / (dn * dn)) / (swv + wd);
+        out[VELX] = (o.su0 + 0.0 / (dn * dn)) / (o.swv + wd);
+        out[VELY] = (o.su1 + 0.0 / (dn * dn)) / (o.swv + wd);
+        out[VELZ] = (o.su2 + 0.0 / (dn * dn)) / (o.swv + wd);
     }
     // homogeneous Neumann IDW of p, T, rho (and species without spec_in_solid), :154-198
-    if (swn > 0.0) {
-        out[PRES] = sp / swn;
-        if (doT) out[TEMP] = sT / swn;
-        out[DENS] = sR / swn;
+    if (o.swn > 0.0) {
+        out[PRES] = o.sp / o.swn;
+        if (doT) out[TEMP] = o.sT / o.swn;
+        out[DENS] = o.sR / o.swn;
         if (doS) {
 #pragma unroll
-            for (int q2 = 0; q2 < NS; ++q2) out[FLO + q2] = sS[q2] / swn;
+            for (int q = 0; q < NS; ++q) out[FLO + q] = o.sS[q] / o.swn;
         }
     }
     if (a.conj_ht) {
@@ -1595,32 +1678,117 @@ __global__ __launch_bounds__(128) void k_cutcells(CutArgs a) {
     // prim_to_cons of the updated primitives (:421-433)
     double u[N::NC], pv[NCV];
 #pragma unroll
-    for (int sp2 = 0; sp2 < NS; ++sp2) u[NCV + sp2] = out[FLO + sp2];
+    for (int q = 0; q < NS; ++q) u[NCV + q] = out[FLO + q];
     pv[0] = out[DENS]; pv[1] = out[VELX]; pv[2] = out[VELY]; pv[3] = out[VELZ]; pv[4] = out[PRES];
     N::prim_to_cons(T, u, pv);
 #pragma unroll
     for (int c = 0; c < NCV; ++c) out[c] = u[c];
+}
+
+// update_cutcells of the level's cut-cell list (ib_utils.H:271-436), 8 lanes
+// per cut cell, with the static geometry and fluid-neighbour mask of k_cut_geom
+template <class P>
+__global__ __launch_bounds__(256) void k_cutcells(CutArgs a) {
+    constexpr int NS = P::NS, NV = Num<P>::NV;
+    if (step_skipped(a.ts)) return;
+    const int lane = threadIdx.x & (kCutLanes - 1);
+    const int q = xcd_chunk(blockIdx.x, gridDim.x) * (256 / kCutLanes) + threadIdx.x / kCutLanes;
+    if (q >= a.ncut) return;
+    const View &s = a.s;
+    const int i = a.list[q], j = a.list[a.ncut + q], k = a.list[2 * a.ncut + q];
+    const double dxmin = fmin(a.dx[0], fmin(a.dx[1], a.dx[2]));
+    const double dnd[3] = {a.dx[0] / dxmin, a.dx[1] / dxmin, a.dx[2] / dxmin};
+    const double xnd[3] = {a.geom[q], a.geom[(int64_t)a.ncut + q], a.geom[(int64_t)2 * a.ncut + q]};
+    const double dist = a.geom[(int64_t)3 * a.ncut + q];
+    const bool vel0 = fabs(dist) < dxmin * 1e-5;
+    CutSums<NS> o = {};
+    for (int r = lane; r < 25; r += kCutLanes) {
+        const int nb = r * 5, w = nb >> 5, sh = nb & 31;
+        unsigned bits = a.mask[(int64_t)w * a.ncut + q] >> sh;
+        if (sh > 27) bits |= a.mask[(int64_t)(w + 1) * a.ncut + q] << (32 - sh);
+        const int m = r % 5 - 2, n = r / 5 - 2;
+        cut_row<NS>(a, s.p + s.off(i, j + m, k + n), m, n, bits & 31u, dnd, xnd, vel0, o);
+    }
+    cut_exchange<NS>(o);
+    if (lane != 0) return;
+    double out[NV];
+    cut_finish<P>(*a.tab, a, i, j, k, dist, vel0, o, out);
 #pragma unroll
     for (int n = 0; n < NV; ++n) a.cutbuf[(int64_t)n * a.ncut + q] = out[n];
 }
 
-// dense form over one box for the per-box C-ABI call: values to tmp, flags set
+// dense form over one box for the per-box C-ABI call: values to tmp, flags
+// set. A block collects the cut cells among its 256 cells and gives each to 8
+// lanes, with the geometry computed on the way: about one cell in eight of a
+// packed bed is cut, and one thread a cell left the others of its wave waiting
+// for 250 serial neighbour reads (123 us for a 32^3 box).
 template <class P>
-__global__ __launch_bounds__(128) void k_cutcells_box(CutArgs a) {
-    constexpr int NV = Num<P>::NV;
+__global__ __launch_bounds__(256) void k_cutcells_box(CutArgs a) {
+    constexpr int NS = P::NS, NV = Num<P>::NV;
+    __shared__ int list[256], count;
     const int ex = a.hi[0] - a.lo[0] + 1, ey = a.hi[1] - a.lo[1] + 1, ez = a.hi[2] - a.lo[2] + 1;
     const int64_t ncell = (int64_t)ex * ey * ez;
-    const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (q >= ncell) return;
-    const int i = a.lo[0] + (int)(q % ex), j = a.lo[1] + (int)((q / ex) % ey), k = a.lo[2] + (int)(q / ((int64_t)ex * ey));
-    const double vf = a.s(i, j, k, VFRAC);
-    const int cut = (vf > kZero && vf < kOne) ? 1 : 0;
-    a.flag[q] = cut;
-    if (!cut) return;
-    double out[NV];
-    cutcell_values<P>(*a.tab, a, i, j, k, out);
+    const int64_t q0 = blockIdx.x * (int64_t)256;
+    const View &s = a.s;
+    auto cell = [&](int64_t q, int &i, int &j, int &k) {
+        i = a.lo[0] + (int)(q % ex);
+        j = a.lo[1] + (int)((q / ex) % ey);
+        k = a.lo[2] + (int)(q / ((int64_t)ex * ey));
+    };
+    if (threadIdx.x == 0) count = 0;
+    __syncthreads();
+    {
+        const int64_t q = q0 + threadIdx.x;
+        bool cut = false;
+        if (q < ncell) {
+            int i, j, k;
+            cell(q, i, j, k);
+            const double vf = s(i, j, k, VFRAC);
+            cut = vf > kZero && vf < kOne;
+            a.flag[q] = cut ? 1 : 0;
+        }
+        if (cut) list[atomicAdd(&count, 1)] = threadIdx.x;
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & (kCutLanes - 1);
+    const double dxmin = fmin(a.dx[0], fmin(a.dx[1], a.dx[2]));
+    const double dnd[3] = {a.dx[0] / dxmin, a.dx[1] / dxmin, a.dx[2] / dxmin};
+    for (int e = threadIdx.x / kCutLanes; e < count; e += 256 / kCutLanes) {
+        const int64_t q = q0 + list[e];
+        int i, j, k;
+        cell(q, i, j, k);
+        const double *c = s.p + s.off(i, j, k) + (int64_t)VFRAC * s.ns;
+        // the level-set gradient of cut_geom_cell: of the 27-point quadratic
+        // basis only the two neighbours along each axis have a weight
+        const double g0 = (c[1] - c[-1]) * (kHalf / a.dx[0]), g1 = (c[s.js] - c[-s.js]) * (kHalf / a.dx[1]),
+                     g2 = (c[s.ks] - c[-s.ks]) * (kHalf / a.dx[2]);
+        const double mag = sqrt(g0 * g0 + g1 * g1 + g2 * g2);
+        double dist = kZero, xnd[3] = {kZero, kZero, kZero};
+        if (mag > kTiny) {
+            dist = (c[0] - kHalf) / mag;
+            xnd[0] = -dist * (g0 / mag) / dxmin;
+            xnd[1] = -dist * (g1 / mag) / dxmin;
+            xnd[2] = -dist * (g2 / mag) / dxmin;
+        }
+        const bool vel0 = fabs(dist) < dxmin * 1e-5;
+        CutSums<NS> o = {};
+        for (int r = lane; r < 25; r += kCutLanes) {
+            const int m = r % 5 - 2, n = r / 5 - 2;
+            const double *row = s.p + s.off(i, j + m, k + n);
+            const double *vf = row + (int64_t)VFRAC * s.ns;
+            unsigned bits = 0u;
 #pragma unroll
-    for (int n = 0; n < NV; ++n) a.tmp[(int64_t)n * ncell + q] = out[n];
+            for (int l = 0; l < 5; ++l) bits |= (vf[l - 2] == 1.0 ? 1u : 0u) << l;
+            cut_row<NS>(a, row, m, n, bits, dnd, xnd, vel0, o);
+        }
+        cut_exchange<NS>(o);
+        if (lane == 0) {
+            double out[NV];
+            cut_finish<P>(*a.tab, a, i, j, k, dist, vel0, o, out);
+#pragma unroll
+            for (int n = 0; n < NV; ++n) a.tmp[(int64_t)n * ncell + q] = out[n];
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1732,14 +1900,20 @@ __global__ __launch_bounds__(256) void k_chem_split(ChemSplitArgs c) {
 
 template <class P>
 struct Launch {
-    static void fill(const FillArgs &a, int phase, hipStream_t st) {
+    // one launch where every rule's source lies inside, else phase by phase
+    static void fill(const FillArgs &a, hipStream_t st) {
         const int G = MF_NGROW;
         int64_t PX = a.n[0] + 2 * G, PY = a.n[1] + 2 * G;
         int64_t total = 2 * G * PX * PY + (int64_t)a.n[2] * 2 * G * PX + (int64_t)a.n[2] * a.n[1] * 2 * G;
         int64_t grid = (total + 255) / 256;
         if (grid > 65535) grid = 65535;
         if (grid < 1) grid = 1;
-        hipLaunchKernelGGL(k_fill<P>, dim3((unsigned)grid), dim3(256), 0, st, a, phase);
+        if (a.n[0] >= G && a.n[1] >= G && a.n[2] >= G) {
+            hipLaunchKernelGGL(k_fill_all<P>, dim3((unsigned)grid), dim3(256), 0, st, a);
+            return;
+        }
+        for (int phase = 0; phase <= 3; ++phase)
+            hipLaunchKernelGGL(k_fill<P>, dim3((unsigned)grid), dim3(256), 0, st, a, phase);
     }
     static void fill_region(const FillArgs &a, int phase, const int *rlo, const int *rhi, hipStream_t st) {
         const int64_t total = (int64_t)(rhi[0] - rlo[0] + 1) * (rhi[1] - rlo[1] + 1) * (rhi[2] - rlo[2] + 1);
@@ -1759,9 +1933,10 @@ struct Launch {
     }
     static void cut(const CutArgs &a, hipStream_t st) {
         if (a.ncut <= 0) return;
-        int g = (a.ncut + 127) / 128;
+        const int per = 256 / kCutLanes;
+        int g = (a.ncut + per - 1) / per;
         if (g >= 8) g = (g + 7) & ~7;
-        hipLaunchKernelGGL(k_cutcells<P>, dim3(g), dim3(128), 0, st, a);
+        hipLaunchKernelGGL(k_cutcells<P>, dim3(g), dim3(256), 0, st, a);
     }
     static void cut_geom(const CutArgs &a, double *geom, unsigned *mask, hipStream_t st) {
         if (a.ncut <= 0) return;
@@ -1774,7 +1949,7 @@ struct Launch {
     static void cut_box(const CutArgs &a, hipStream_t st) {
         int64_t n = (int64_t)(a.hi[0] - a.lo[0] + 1) * (a.hi[1] - a.lo[1] + 1) * (a.hi[2] - a.lo[2] + 1);
         if (n <= 0) return;
-        hipLaunchKernelGGL(k_cutcells_box<P>, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, st, a);
+        hipLaunchKernelGGL(k_cutcells_box<P>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a);
     }
     template <int ORDER>
     static void faces_o(const StageArgs &a, const Work &w, int dir, int grid, int block, hipStream_t st) {
@@ -1794,7 +1969,7 @@ struct Launch {
         int e[3] = {tsh[0], tsh[1], tsh[2]};
         e[dir] += 6;
         const size_t ncs = (size_t)e[0] * e[1] * e[2];
-        return ncs * ((Num<P>::NC + 6) | 1) * sizeof(double) + ((ncs * sizeof(int) + 7) & ~(size_t)7);
+        return ncs * kFaceRec<P> * sizeof(double) + ((ncs * sizeof(int) + 7) & ~(size_t)7);
     }
     static void faces_lds(const StageArgs &a, const Work &w, int dir, int grid, int block, size_t lds, hipStream_t st) {
         static bool attr = false;
