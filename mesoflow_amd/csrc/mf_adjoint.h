@@ -852,6 +852,31 @@ struct Rev {
             for (int s = 0; s < NS; ++s) lint[FLO + s] += specb[s];
         }
     }
+    // adjoint of fill_value<P, true>: l, the adjoint of ghost cell c, becomes
+    // the adjoint of the valid cell that c becomes; the state a.s is the filled one
+    MFD static void fill_rev(const Tab &T, const FillArgs &a, int *c, double *l, double &invelb) {
+        FillRule r;
+        while (fill_rule(a, c, r)) {
+            fill_source(a, r, c);
+            if (r.bc == MF_BC_EXT_DIR) {
+                double s_int[NV], lint[NV];
+                const double *src = a.s.p + a.s.off(c[0], c[1], c[2]);
+#pragma unroll
+                for (int n = 0; n < NV; ++n) {
+                    s_int[n] = src[(int64_t)n * a.s.ns];
+                    lint[n] = 0.0;
+                }
+                externalbc_rev(T, s_int, l, r.d, r.low ? 1 : -1, lint, invelb);
+#pragma unroll
+                for (int n = 0; n < NV; ++n) l[n] = lint[n];
+            } else if (r.bc == MF_BC_WALL) {
+#pragma unroll
+                for (int n = 0; n < NV; ++n)
+                    if (wall_odd(n)) l[n] = -l[n];
+            }
+        }
+        fill_wrap(a, c);
+    }
 };
 
 }  // namespace mfd

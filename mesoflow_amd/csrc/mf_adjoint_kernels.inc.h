@@ -4,7 +4,7 @@
 // stage in reverse order:
 //   k_faces_adj (x, y, z)  adjoint of the face fluxes and update_residual
 //   k_cut_adj              adjoint of update_cutcells
-//   k_fill_adj (3, 2, 1, 0) adjoint of the ghost fill
+//   k_fill_adj              adjoint of the ghost fill
 // after k_post_adj (adjoint of chemistry, update_primitive_vars, clip and of
 // the objective's outlet term of the step).
 #pragma once
@@ -325,10 +325,12 @@ __global__ __launch_bounds__(128) void k_cut_gather(AdjCutArgs aa) {
         if (res[6 + s] != 0.0) lam(i, j, k, FLO + s) += res[6 + s];
 }
 
-// adjoint of one phase of k_fill: ghost adjoints go to the cells the ghost was
-// filled from (the last rule that wrote it) and are cleared
+// adjoint of k_fill: the adjoint of a ghost cell goes along its chain of rules
+// to the valid cell the chain ends at and is cleared. A thread writes its own
+// ghost cell and adds to valid cells only, so the order of the ghost cells does
+// not matter; the states that externalbc's adjoint reads are the filled ones.
 template <class P>
-__global__ __launch_bounds__(256) void k_fill_adj(AdjFillArgs aa, int phase) {
+__global__ __launch_bounds__(256) void k_fill_adj(AdjFillArgs aa) {
     constexpr int NV = Num<P>::NV;
     const FillArgs &a = aa.f;
     if (step_skipped(a.ts)) return;
@@ -343,85 +345,20 @@ __global__ __launch_bounds__(256) void k_fill_adj(AdjFillArgs aa, int phase) {
     const int64_t total = nzs + nys + nxs;
     double invelb = 0.0;
     for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
-        int iv[3];
-        if (q < nzs) {
-            int64_t r = q;
-            iv[0] = (int)(r % PX) - G; r /= PX;
-            iv[1] = (int)(r % PY) - G; r /= PY;
-            int g = (int)r;
-            iv[2] = g < G ? g - G : nz + (g - G);
-        } else if (q < nzs + nys) {
-            int64_t r = q - nzs;
-            iv[0] = (int)(r % PX) - G; r /= PX;
-            int g = (int)(r % (2 * G)); r /= (2 * G);
-            iv[1] = g < G ? g - G : ny + (g - G);
-            iv[2] = (int)r;
-        } else {
-            int64_t r = q - nzs - nys;
-            int g = (int)(r % (2 * G)); r /= (2 * G);
-            iv[0] = g < G ? g - G : nx + (g - G);
-            iv[1] = (int)(r % ny); r /= ny;
-            iv[2] = (int)r;
-        }
-        int out_np = 0, out_p = 0;
+        int c[3];
+        ghost_cell(q, nzs, nys, PX, PY, nx, ny, nz, c);
+        double l[NV];
+        double *g = lam.p + lam.off(c[0], c[1], c[2]);
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            bool o = iv[d] < 0 || iv[d] >= a.n[d];
-            if (o) { if (a.periodic[d]) ++out_p; else ++out_np; }
+        for (int n = 0; n < NV; ++n) {
+            l[n] = g[(int64_t)n * lam.ns];
+            g[(int64_t)n * lam.ns] = 0.0;
         }
-        if (phase == 0) {
-            if (out_np != 0 || out_p == 0) continue;
-            int s[3];
+        Rev<P>::fill_rev(T, a, c, l, invelb);
+        double *to = lam.p + lam.off(c[0], c[1], c[2]);
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                s[d] = iv[d];
-                if (a.periodic[d]) { if (s[d] < 0) s[d] += a.n[d]; else if (s[d] >= a.n[d]) s[d] -= a.n[d]; }
-            }
-            for (int c = 0; c < NV; ++c) {
-                const double v = lam(iv[0], iv[1], iv[2], c);
-                if (v != 0.0) unsafeAtomicAdd(&lam(s[0], s[1], s[2], c), v);
-                lam(iv[0], iv[1], iv[2], c) = 0.0;
-            }
-            continue;
-        }
-        if (out_np != phase) continue;
-        int ext = -1, sgn = 0, bnd = 0, fil = -1;
-        for (int d = 0; d < 3; ++d) {
-            if (a.periodic[d]) continue;
-            if (a.lo_bc[d] == MF_BC_EXT_DIR && iv[d] < 0) { ext = d; sgn = 1; bnd = 0; }
-            else if (a.hi_bc[d] == MF_BC_EXT_DIR && iv[d] >= a.n[d]) { ext = d; sgn = -1; bnd = a.n[d] - 1; }
-            const int side = iv[d] < 0 ? 0 : (iv[d] >= a.n[d] ? 1 : -1);
-            if (side >= 0 && (side == 0 ? a.lo_bc[d] : a.hi_bc[d]) != MF_BC_EXT_DIR) fil = d;
-        }
-        if (ext >= 0) {
-            int loc[3] = {iv[0], iv[1], iv[2]};
-            loc[ext] = bnd;
-            double s_int[NV], lext[NV], lint[NV];
-            for (int c = 0; c < NV; ++c) {
-                s_int[c] = a.s(loc[0], loc[1], loc[2], c);
-                lext[c] = lam(iv[0], iv[1], iv[2], c);
-                lint[c] = 0.0;
-            }
-            Rev<P>::externalbc_rev(T, s_int, lext, ext, sgn, lint, invelb);
-            for (int c = 0; c < NV; ++c) {
-                if (lint[c] != 0.0) unsafeAtomicAdd(&lam(loc[0], loc[1], loc[2], c), lint[c]);
-                lam(iv[0], iv[1], iv[2], c) = 0.0;
-            }
-        } else if (fil >= 0) {
-            const int d = fil;
-            const int side = iv[d] < 0 ? 0 : 1;
-            const int bc = side == 0 ? a.lo_bc[d] : a.hi_bc[d];
-            int s[3] = {iv[0], iv[1], iv[2]};
-            const bool refl = (bc == MF_BC_WALL);
-            if (!refl) s[d] = side == 0 ? 0 : a.n[d] - 1;
-            else s[d] = side == 0 ? (-iv[d] - 1) : (2 * (a.n[d] - 1) - iv[d] + 1);
-            for (int c = 0; c < NV; ++c) {
-                const double v = lam(iv[0], iv[1], iv[2], c);
-                const bool odd = refl && (c == RHOU || c == RHOV || c == RHOW || c == VELX || c == VELY || c == VELZ);
-                if (v != 0.0) unsafeAtomicAdd(&lam(s[0], s[1], s[2], c), odd ? -v : v);
-                lam(iv[0], iv[1], iv[2], c) = 0.0;
-            }
-        }
+        for (int n = 0; n < NV; ++n)
+            if (l[n] != 0.0) unsafeAtomicAdd(to + (int64_t)n * lam.ns, l[n]);
     }
     if (invelb != 0.0) unsafeAtomicAdd(aa.grad + T.nreact, invelb);
 }
@@ -533,14 +470,14 @@ struct AdjLaunch {
         hipLaunchKernelGGL(k_cut_coef<P>, dim3(cut_grid(a.c.ncut)), dim3(128), 0, st, a);
         if (a.nnbr > 0) hipLaunchKernelGGL(k_cut_gather<P>, dim3(cut_grid(a.nnbr)), dim3(128), 0, st, a);
     }
-    static void fill(const AdjFillArgs &a, int phase, hipStream_t st) {
+    static void fill(const AdjFillArgs &a, hipStream_t st) {
         const int G = MF_NGROW;
         int64_t PX = a.f.n[0] + 2 * G, PY = a.f.n[1] + 2 * G;
         int64_t total = 2 * G * PX * PY + (int64_t)a.f.n[2] * 2 * G * PX + (int64_t)a.f.n[2] * a.f.n[1] * 2 * G;
         int64_t grid = (total + 255) / 256;
         if (grid > 65535) grid = 65535;
         if (grid < 1) grid = 1;
-        hipLaunchKernelGGL(k_fill_adj<P>, dim3((unsigned)grid), dim3(256), 0, st, a, phase);
+        hipLaunchKernelGGL(k_fill_adj<P>, dim3((unsigned)grid), dim3(256), 0, st, a);
     }
     static void post(const AdjPostArgs &a, const Work &w, int grid, int block, hipStream_t st) {
         hipLaunchKernelGGL(k_post_adj<P>, dim3(grid), dim3(block), 0, st, a, w);

@@ -161,7 +161,7 @@ struct AdjSet {
     void (*faces)(const AdjFaceArgs &, const Work &, int dir, int grid, int block, size_t lds, hipStream_t);
     size_t (*lds_bytes)(const int *tsh, int dir);
     void (*cut)(const AdjCutArgs &, hipStream_t);
-    void (*fill)(const AdjFillArgs &, int phase, hipStream_t);
+    void (*fill)(const AdjFillArgs &, hipStream_t);
     void (*post)(const AdjPostArgs &, const Work &, int grid, int block, hipStream_t);
     void (*objective)(const ObjArgs &, hipStream_t);
     int cut_rec;               // doubles per cut-cell record of AdjCutArgs::coef
@@ -197,10 +197,10 @@ struct KernelSet {
     int ns;
     bool has_bg_gas;           // the family's thermo has a background gas (using_bg_inertgas)
     void (*fill)(const FillArgs &, hipStream_t);
-    // physical-boundary phase of the fill over the region [rlo, rhi] of a.s
-    void (*fill_region)(const FillArgs &, int phase, const int *rlo, const int *rhi, hipStream_t);
-    // physical-boundary phase of the fill over a list of cells ([3][n])
-    void (*fill_list)(const FillArgs &, int phase, const int *list, int n, hipStream_t);
+    // physical-boundary rules of the fill over the region [rlo, rhi] of a.s
+    void (*fill_region)(const FillArgs &, const int *rlo, const int *rhi, hipStream_t);
+    // the same over a list of cells ([3][n])
+    void (*fill_list)(const FillArgs &, const int *list, int n, hipStream_t);
     // chemistry alone over the tile list (st.src -> dst)
     void (*chem)(const ResArgs &, const Work &, int grid, int block, hipStream_t);
     void (*cut)(const CutArgs &, hipStream_t);

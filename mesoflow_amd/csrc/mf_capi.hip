@@ -1061,7 +1061,7 @@ void adj_stage_reverse(Level *L, int stage, View lam_out, double coef, double *l
     fl.f = fill_args(L, src, stage);
     fl.lam = lin;
     fl.grad = A->grad;
-    for (int ph = 3; ph >= 0; --ph) S->fill(fl, ph, c->stream);
+    S->fill(fl, c->stream);
 }
 
 // adjoint of step n: A holds U^n; lam[0] holds the adjoint of U^{n+1} on entry
@@ -2356,9 +2356,8 @@ int mf_ctx_aux(void *ctx, size_t bytes, double **p) {
 
 // the physical-boundary rules of the single-level fill (foextrap, wall
 // reflection, the plugin's externalbc; Source/mflo_bcfill.H:16-128) on the
-// cells of `region` of `view` outside the domain in non-periodic directions,
-// in phases of 1, 2, 3 such directions; every other cell of the region must
-// be filled already. For mf_amr.hip (FillPatchTwoLevels of a fine box).
+// cells of `region` of `view` outside the domain in non-periodic directions;
+// every other cell of the region must be filled already. For mf_amr.hip (FillPatchTwoLevels of a fine box).
 int mf_ctx_fill_physbc(void *ctx, mf_array4 view, mf_box region, double time) {
     Ctx *c = (Ctx *)ctx;
     if (!c || !view.p || view.ncomp < c->nv) return MF_ERR_BAD_ARG;
@@ -2384,7 +2383,7 @@ int mf_ctx_fill_physbc(void *ctx, mf_array4 view, mf_box region, double time) {
     f.ts = nullptr;
     f.time_host = time;
     f.stage = 1;
-    for (int ph = 1; ph <= 3; ++ph) c->ks->fill_region(f, ph, region.lo, region.hi, c->stream);
+    c->ks->fill_region(f, region.lo, region.hi, c->stream);
     HIPCHK(hipGetLastError());
     return MF_OK;
 }

@@ -660,7 +660,7 @@ void hier_fill_fine(Hier *H, double *dst, double *c_old, double *c_new, int stag
                            Lf->n[0], Lf->n[1], Lf->n[2], ts0);
     FillArgs ff = fill_args(Lf, dst, stage);
     ff.ts = Lf->ts;
-    for (int ph = 1; ph <= 3; ++ph) cf->ks->fill_list(ff, ph, H->fphys[ph - 1], H->nfphys[ph - 1], st);
+    for (int ph = 1; ph <= 3; ++ph) cf->ks->fill_list(ff, H->fphys[ph - 1], H->nfphys[ph - 1], st);
 }
 
 // one RK3 stage of a level of the hierarchy (Advance_coupled_strang

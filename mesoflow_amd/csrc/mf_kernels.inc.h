@@ -1134,67 +1134,100 @@ __global__ __launch_bounds__(256) void k_est(ResArgs r, Work w) {
 }
 
 // ---------------------------------------------------------------------------
-// Ghost cells of the padded level array (FillPatchSingleLevel): phase 0 fills
-// cells outside only in periodic directions from their periodic images; phase
-// p >= 1 fills cells outside in p non-periodic directions with the filcc rules
-// (foextrap, reflect_even/odd for walls: Source/mflo.cpp:70-143) in x,y,z order,
-// then the ext_dir functor of Source/mflo_bcfill.H:16-128 in x,y,z order.
+// Ghost cells of the padded level array (FillPatchSingleLevel). A cell outside
+// the domain in a non-periodic direction takes one rule: the ext_dir functor of
+// Source/mflo_bcfill.H:16-128 in the last direction that has one, else the
+// filcc rule of the last direction (foextrap, reflect_even/odd for walls:
+// Source/mflo.cpp:70-143), since x, y and z are applied in that order and the
+// functor after filcc. A rule reads the cell it is filled from, which may lie
+// outside in another direction, or, past a wall of a domain thinner than the
+// ghost layer, beyond the opposite side: the rules of a ghost cell form a chain
+// that ends at a cell outside in periodic directions at most.
 // ---------------------------------------------------------------------------
-// the rules of one ghost cell iv of a.s for the given phase (cells outside the
-// domain in phase non-periodic directions; phase 0: only in periodic ones)
-template <class P>
-MFD void fill_cell_rules(const FillArgs &a, const int *iv, int phase, const Tab &T, double time) {
+struct FillRule { int d, low, bc; };
+// the rule of cell c, false where c lies inside in every non-periodic direction
+MFD bool fill_rule(const FillArgs &a, const int *c, FillRule &r) {
+    r.d = -1;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (a.periodic[d] || (c[d] >= 0 && c[d] < a.n[d])) continue;
+        const int bc = c[d] < 0 ? a.lo_bc[d] : a.hi_bc[d];
+        if (bc != MF_BC_EXT_DIR && r.d >= 0 && r.bc == MF_BC_EXT_DIR) continue;
+        r.d = d;
+        r.low = c[d] < 0;
+        r.bc = bc;
+    }
+    return r.d >= 0;
+}
+// c becomes the cell that rule r of c reads: the edge cell, or the mirror image
+// of a wall (which moves a cell past both walls of a thin domain ever closer)
+MFD void fill_source(const FillArgs &a, const FillRule &r, int *c) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (d != r.d) continue;
+        if (r.bc == MF_BC_WALL) c[d] = r.low ? -c[d] - 1 : 2 * (a.n[d] - 1) - c[d] + 1;
+        else c[d] = r.low ? 0 : a.n[d] - 1;
+    }
+}
+// the periodic image of c inside the domain, for any number of cells
+MFD void fill_wrap(const FillArgs &a, int *c) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (!a.periodic[d]) continue;
+        while (c[d] < 0) c[d] += a.n[d];
+        while (c[d] >= a.n[d]) c[d] -= a.n[d];
+    }
+}
+MFD bool wall_odd(int n) { return n == RHOU || n == RHOV || n == RHOW || n == VELX || n == VELY || n == VELZ; }
+
+// the value of ghost cell iv: the chain is walked to its last cell, whose
+// values then take the rules on the way back (rule s is found by walking s
+// steps again: nearly every chain has one or two). Only that last cell is read, with WRAP a
+// valid cell, so no ghost cell waits for another one.
+template <class P, bool WRAP>
+MFD void fill_value(const FillArgs &a, const int *iv, const Tab &T, double time, double *v) {
     constexpr int NV = Num<P>::NV;
-    int out_np = 0, out_p = 0;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        bool o = iv[d] < 0 || iv[d] >= a.n[d];
-        if (o) { if (a.periodic[d]) ++out_p; else ++out_np; }
+    int c[3] = {iv[0], iv[1], iv[2]}, nr = 0;
+    FillRule r;
+    while (fill_rule(a, c, r)) {
+        fill_source(a, r, c);
+        ++nr;
     }
-    if (phase == 0) {
-        if (out_np != 0 || out_p == 0) return;
-        int s[3];
+    if (WRAP) fill_wrap(a, c);
+    const double *src = a.s.p + a.s.off(c[0], c[1], c[2]);
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            s[d] = iv[d];
-            if (a.periodic[d]) { if (s[d] < 0) s[d] += a.n[d]; else if (s[d] >= a.n[d]) s[d] -= a.n[d]; }
+    for (int n = 0; n < NV; ++n) v[n] = src[(int64_t)n * a.s.ns];
+    for (int s = nr - 1; s >= 0; --s) {
+        int p[3] = {iv[0], iv[1], iv[2]};
+        fill_rule(a, p, r);
+        for (int q = 0; q < s; ++q) {
+            fill_source(a, r, p);
+            fill_rule(a, p, r);
         }
-        for (int c = 0; c < NV; ++c) a.s(iv[0], iv[1], iv[2], c) = a.s(s[0], s[1], s[2], c);
-        return;
-    }
-    if (out_np != phase) return;
-    for (int d = 0; d < 3; ++d) {
-        if (a.periodic[d]) continue;
-        int side = iv[d] < 0 ? 0 : (iv[d] >= a.n[d] ? 1 : -1);
-        if (side < 0) continue;
-        int bc = side == 0 ? a.lo_bc[d] : a.hi_bc[d];
-        if (bc == MF_BC_EXT_DIR) continue;
-        int s[3] = {iv[0], iv[1], iv[2]};
-        bool refl = (bc == MF_BC_WALL);
-        if (!refl) s[d] = side == 0 ? 0 : a.n[d] - 1;
-        else s[d] = side == 0 ? (-iv[d] - 1) : (2 * (a.n[d] - 1) - iv[d] + 1);
-        for (int c = 0; c < NV; ++c) {
-            double v = a.s(s[0], s[1], s[2], c);
-            bool odd = refl && (c == RHOU || c == RHOV || c == RHOW || c == VELX || c == VELY || c == VELZ);
-            a.s(iv[0], iv[1], iv[2], c) = odd ? -v : v;
+        if (r.bc == MF_BC_EXT_DIR) {
+            double x[3], e[NV];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) x[d] = a.prob_lo[d] + (p[d] + 0.5) * a.dx[d];
+#pragma unroll
+            for (int n = 0; n < NV; ++n) e[n] = 0.0;
+            P::externalbc(T, x, v, e, r.d, r.low ? 1 : -1, time);
+#pragma unroll
+            for (int n = 0; n < NV; ++n) v[n] = e[n];
+        } else if (r.bc == MF_BC_WALL) {
+#pragma unroll
+            for (int n = 0; n < NV; ++n)
+                if (wall_odd(n)) v[n] = -v[n];
         }
     }
-    double x[3];
+}
+template <class P, bool WRAP>
+MFD void fill_cell(const FillArgs &a, const int *iv, const Tab &T, double time) {
+    constexpr int NV = Num<P>::NV;
+    double v[NV];
+    fill_value<P, WRAP>(a, iv, T, time, v);
+    double *dst = a.s.p + a.s.off(iv[0], iv[1], iv[2]);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) x[d] = a.prob_lo[d] + (iv[d] + 0.5) * a.dx[d];
-    for (int d = 0; d < 3; ++d) {
-        if (a.periodic[d]) continue;
-        int sgn = 0, bnd = 0;
-        if (a.lo_bc[d] == MF_BC_EXT_DIR && iv[d] < 0) { sgn = 1; bnd = 0; }
-        else if (a.hi_bc[d] == MF_BC_EXT_DIR && iv[d] >= a.n[d]) { sgn = -1; bnd = a.n[d] - 1; }
-        if (!sgn) continue;
-        double s_int[NV], s_ext[NV];
-        int loc[3] = {iv[0], iv[1], iv[2]};
-        loc[d] = bnd;
-        for (int c = 0; c < NV; ++c) { s_int[c] = a.s(loc[0], loc[1], loc[2], c); s_ext[c] = 0.0; }
-        P::externalbc(T, x, s_int, s_ext, d, sgn, time);
-        for (int c = 0; c < NV; ++c) a.s(iv[0], iv[1], iv[2], c) = s_ext[c];
-    }
+    for (int n = 0; n < NV; ++n) dst[(int64_t)n * a.s.ns] = v[n];
 }
 
 // ghost cell q of a padded level array: the z slabs, then the y slabs of the
@@ -1222,8 +1255,12 @@ MFD void ghost_cell(int64_t q, int64_t nzs, int64_t nys, int PX, int PY, int nx,
     }
 }
 
+// the ghost cells of a padded level array in one launch: bound by launches at
+// small sizes, by the reads of the domain shell at large ones (12 us a fill at
+// 64^3 and 108 us at 256^3 with 17 components, timed between events that cost 6;
+// four launches, one per number of outside directions, took 27 and 162)
 template <class P>
-__global__ __launch_bounds__(256) void k_fill(FillArgs a, int phase) {
+__global__ __launch_bounds__(256) void k_fill(FillArgs a) {
     if (step_skipped(a.ts)) return;
     const Tab &T = *a.tab;
     const double time = !a.ts ? a.time_host : (a.stage == 1 ? a.ts->t : a.ts->t + a.ts->dt);
@@ -1237,106 +1274,17 @@ __global__ __launch_bounds__(256) void k_fill(FillArgs a, int phase) {
     for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
         int iv[3];
         ghost_cell(q, nzs, nys, PX, PY, nx, ny, nz, iv);
-        fill_cell_rules<P>(a, iv, phase, T, time);
+        fill_cell<P, true>(a, iv, T, time);
     }
 }
 
-// All phases of k_fill in one launch. The rule that decides a ghost cell (the
-// last ext_dir direction it lies outside of, else the last foextrap or wall
-// one) reads a cell with one outside direction fewer, so every ghost cell is a
-// chain of at most three rules over one valid cell: the chain is walked to that
-// cell and its rules are applied on the way back, with the arithmetic of the
-// phases. It reads valid cells only (no order between ghost cells) and needs
-// every rule's source one step inside: at least MF_NGROW cells per direction.
-// Bound by launches at small sizes: four dependent launches a stage became one
-// (19 -> 6 us a stage for 32x4x4 cells).
+// The physical-boundary rules over the cells of the region [rlo, rhi] of a.s
+// that lie outside the domain in a non-periodic direction: the ghost region of
+// a box whose other cells are already filled (FillPatchTwoLevels' physical
+// boundary fill of a fine box). A chain's last cell is one of those others: it
+// lies inside any box grown by 3 that reaches beyond the domain.
 template <class P>
-__global__ __launch_bounds__(256) void k_fill_all(FillArgs a) {
-    constexpr int NV = Num<P>::NV;
-    if (step_skipped(a.ts)) return;
-    const Tab &T = *a.tab;
-    const double time = !a.ts ? a.time_host : (a.stage == 1 ? a.ts->t : a.ts->t + a.ts->dt);
-    const int G = MF_NGROW;
-    const int nx = a.n[0], ny = a.n[1], nz = a.n[2];
-    const int PX = nx + 2 * G, PY = ny + 2 * G;
-    const int64_t nzs = (int64_t)2 * G * PX * PY;
-    const int64_t nys = (int64_t)nz * 2 * G * PX;
-    const int64_t nxs = (int64_t)nz * ny * 2 * G;
-    const int64_t total = nzs + nys + nxs;
-    for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
-        int iv[3];
-        ghost_cell(q, nzs, nys, PX, PY, nx, ny, nz, iv);
-        // the chain: the direction of each rule and the position it applies at
-        int at[3][3], dir[3], nr = 0, c[3] = {iv[0], iv[1], iv[2]};
-#pragma unroll
-        for (int step = 0; step < 3; ++step) {
-            int pick = -1;
-            bool ext = false;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                if (a.periodic[d] || (c[d] >= 0 && c[d] < a.n[d])) continue;
-                const bool e = (c[d] < 0 ? a.lo_bc[d] : a.hi_bc[d]) == MF_BC_EXT_DIR;
-                if (e || !ext) { pick = d; ext = e; }
-            }
-            if (pick < 0) break;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) at[step][d] = c[d];
-            dir[step] = pick;
-            nr = step + 1;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                if (d != pick) continue;
-                const bool low = c[d] < 0;
-                const int bc = low ? a.lo_bc[d] : a.hi_bc[d];
-                if (bc == MF_BC_WALL) c[d] = low ? -c[d] - 1 : 2 * (a.n[d] - 1) - c[d] + 1;
-                else c[d] = low ? 0 : a.n[d] - 1;
-            }
-        }
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            if (c[d] < 0) c[d] += a.n[d];
-            else if (c[d] >= a.n[d]) c[d] -= a.n[d];
-        }
-        double v[NV];
-        const double *src = a.s.p + a.s.off(c[0], c[1], c[2]);
-#pragma unroll
-        for (int n = 0; n < NV; ++n) v[n] = src[(int64_t)n * a.s.ns];
-#pragma unroll
-        for (int step = 2; step >= 0; --step) {
-            if (step >= nr) continue;
-            const int d = dir[step];
-            const int pd = d == 0 ? at[step][0] : (d == 1 ? at[step][1] : at[step][2]);
-            const bool low = pd < 0;
-            const int bc = low ? a.lo_bc[d] : a.hi_bc[d];
-            if (bc == MF_BC_EXT_DIR) {
-                double x[3], e[NV];
-#pragma unroll
-                for (int m = 0; m < 3; ++m) x[m] = a.prob_lo[m] + (at[step][m] + 0.5) * a.dx[m];
-#pragma unroll
-                for (int n = 0; n < NV; ++n) e[n] = 0.0;
-                P::externalbc(T, x, v, e, d, low ? 1 : -1, time);
-#pragma unroll
-                for (int n = 0; n < NV; ++n) v[n] = e[n];
-            } else if (bc == MF_BC_WALL) {
-#pragma unroll
-                for (int n = 0; n < NV; ++n)
-                    if (n == RHOU || n == RHOV || n == RHOW || n == VELX || n == VELY || n == VELZ) v[n] = -v[n];
-            }
-        }
-        double *dst = a.s.p + a.s.off(iv[0], iv[1], iv[2]);
-#pragma unroll
-        for (int n = 0; n < NV; ++n) dst[(int64_t)n * a.s.ns] = v[n];
-    }
-}
-
-// The physical-boundary rules (phases >= 1) over the cells of the region
-// [rlo, rhi] of a.s that lie outside the domain: the ghost region of a box
-// whose other cells are already filled (FillPatchTwoLevels' physical boundary
-// fill of a fine box). Each rule reads only cells of the region: the source
-// planes 0..2 and n-3..n-1 lie inside any box grown by 3 that reaches beyond
-// the domain.
-template <class P>
-__global__ __launch_bounds__(256) void k_fill_region(FillArgs a, int phase, int3 rlo, int3 rhi) {
+__global__ __launch_bounds__(256) void k_fill_region(FillArgs a, int3 rlo, int3 rhi) {
     const Tab &T = *a.tab;
     const double time = a.time_host;
     const int ex = rhi.x - rlo.x + 1, ey = rhi.y - rlo.y + 1, ez = rhi.z - rlo.z + 1;
@@ -1347,23 +1295,22 @@ __global__ __launch_bounds__(256) void k_fill_region(FillArgs a, int phase, int3
         iv[0] = rlo.x + (int)(r % ex); r /= ex;
         iv[1] = rlo.y + (int)(r % ey); r /= ey;
         iv[2] = rlo.z + (int)r;
-        fill_cell_rules<P>(a, iv, phase, T, time);
+        FillRule f;
+        if (fill_rule(a, iv, f)) fill_cell<P, false>(a, iv, T, time);
     }
 }
 
-// The rules of one phase over a list of cells of a.s ([3][n]: i, j, k), the
-// ghost cells of a partly covered level that lie outside the domain
-// (FillPatchTwoLevels' physical boundary fill of the fine boxes); the sources
-// of a phase are cells of earlier phases or interior cells, so the cells of a
-// phase are independent.
+// The same over a list of cells of a.s ([3][n]: i, j, k), the ghost cells of a
+// partly covered level that lie outside the domain (FillPatchTwoLevels'
+// physical boundary fill of the fine boxes)
 template <class P>
-__global__ __launch_bounds__(256) void k_fill_list(FillArgs a, int phase, const int *list, int n) {
+__global__ __launch_bounds__(256) void k_fill_list(FillArgs a, const int *list, int n) {
     if (step_skipped(a.ts)) return;
     const Tab &T = *a.tab;
     const double time = !a.ts ? a.time_host : (a.stage == 1 ? a.ts->t : a.ts->t + a.ts->dt);
     for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) {
         const int iv[3] = {list[q], list[n + q], list[2 * n + q]};
-        fill_cell_rules<P>(a, iv, phase, T, time);
+        fill_cell<P, false>(a, iv, T, time);
     }
 }
 
@@ -1900,7 +1847,6 @@ __global__ __launch_bounds__(256) void k_chem_split(ChemSplitArgs c) {
 
 template <class P>
 struct Launch {
-    // one launch where every rule's source lies inside, else phase by phase
     static void fill(const FillArgs &a, hipStream_t st) {
         const int G = MF_NGROW;
         int64_t PX = a.n[0] + 2 * G, PY = a.n[1] + 2 * G;
@@ -1908,25 +1854,20 @@ struct Launch {
         int64_t grid = (total + 255) / 256;
         if (grid > 65535) grid = 65535;
         if (grid < 1) grid = 1;
-        if (a.n[0] >= G && a.n[1] >= G && a.n[2] >= G) {
-            hipLaunchKernelGGL(k_fill_all<P>, dim3((unsigned)grid), dim3(256), 0, st, a);
-            return;
-        }
-        for (int phase = 0; phase <= 3; ++phase)
-            hipLaunchKernelGGL(k_fill<P>, dim3((unsigned)grid), dim3(256), 0, st, a, phase);
+        hipLaunchKernelGGL(k_fill<P>, dim3((unsigned)grid), dim3(256), 0, st, a);
     }
-    static void fill_region(const FillArgs &a, int phase, const int *rlo, const int *rhi, hipStream_t st) {
+    static void fill_region(const FillArgs &a, const int *rlo, const int *rhi, hipStream_t st) {
         const int64_t total = (int64_t)(rhi[0] - rlo[0] + 1) * (rhi[1] - rlo[1] + 1) * (rhi[2] - rlo[2] + 1);
         if (total <= 0) return;
         int64_t grid = (total + 255) / 256;
         if (grid > 65535) grid = 65535;
-        hipLaunchKernelGGL(k_fill_region<P>, dim3((unsigned)grid), dim3(256), 0, st, a, phase,
+        hipLaunchKernelGGL(k_fill_region<P>, dim3((unsigned)grid), dim3(256), 0, st, a,
                            make_int3(rlo[0], rlo[1], rlo[2]), make_int3(rhi[0], rhi[1], rhi[2]));
     }
-    static void fill_list(const FillArgs &a, int phase, const int *list, int n, hipStream_t st) {
+    static void fill_list(const FillArgs &a, const int *list, int n, hipStream_t st) {
         if (n <= 0) return;
         const int grid = std::min((n + 255) / 256, 65535);
-        hipLaunchKernelGGL(k_fill_list<P>, dim3((unsigned)grid), dim3(256), 0, st, a, phase, list, n);
+        hipLaunchKernelGGL(k_fill_list<P>, dim3((unsigned)grid), dim3(256), 0, st, a, list, n);
     }
     static void chem(const ResArgs &r, const Work &w, int grid, int block, hipStream_t st) {
         hipLaunchKernelGGL(k_chem_tiles<P>, dim3(grid), dim3(block), 0, st, r, w);

@@ -1107,13 +1107,14 @@ struct Level : LevelBase {
                         int s[3];
                         for (int d = 0; d < 3; ++d) {
                             s[d] = iv[d];
-                            if (per[d]) { if (s[d] < 0) s[d] += n[d]; else if (s[d] >= n[d]) s[d] -= n[d]; }
+                            if (per[d]) s[d] = ((s[d] % n[d]) + n[d]) % n[d];  // thin domains: several periods away
                         }
                         for (int c = 0; c < NV; ++c) F(i, j, k, c) = F(s[0], s[1], s[2], c);
                     }
                 }
+        const bool thin = n[0] < 3 || n[1] < 3 || n[2] < 3;  // fill_cell then fills other cells of its phase too
         for (int phase = 1; phase <= 3; ++phase) {
-#pragma omp parallel for schedule(static)
+#pragma omp parallel for schedule(static) if (!thin)
             for (int k = -3; k < n[2] + 3; ++k)
                 for (int j = -3; j < n[1] + 3; ++j)
                     for (int i = -3; i < n[0] + 3; ++i) {
@@ -1134,6 +1135,13 @@ struct Level : LevelBase {
             if (side < 0) continue;
             int bc = side == 0 ? prm.lo_bc[d] : prm.hi_bc[d];
             if (bc == MF_BC_EXT_DIR) continue;
+            if (bc == MF_BC_WALL) {
+                // past a wall of a domain thinner than the ghost layer the mirror
+                // image is itself a ghost cell beyond the opposite side, filled first
+                int m[3] = {iv[0], iv[1], iv[2]};
+                m[d] = side == 0 ? (2 * lo[d] - iv[d] - 1) : (2 * hi[d] - iv[d] + 1);
+                if (m[d] < lo[d] || m[d] > hi[d]) fill_cell(F, m, time);
+            }
             for (int c = 0; c < NV; ++c) {
                 int s[3] = {iv[0], iv[1], iv[2]};
                 double sign = 1.0;
