@@ -612,29 +612,10 @@ struct Rev {
             cutcell_values<P>(T, a, i, j, k, out);
         }
         const double *dx = a.dx;
-        double lsg[3] = {0.0, 0.0, 0.0};
-        const double zero = 0.0;
-        for (int n = -1; n <= 1; n++)
-            for (int m = -1; m <= 1; m++)
-                for (int l = -1; l <= 1; l++) {
-                    double v = s(i + l, j + m, k + n, VFRAC);
-                    double bx = ib_basisder1d(l, zero / dx[0]) / dx[0] * ib_basis1d(m, zero / dx[1]) * ib_basis1d(n, zero / dx[2]);
-                    double by = ib_basis1d(l, zero / dx[0]) * (ib_basisder1d(m, zero / dx[1]) / dx[1]) * ib_basis1d(n, zero / dx[2]);
-                    double bz = ib_basis1d(l, zero / dx[0]) * ib_basis1d(m, zero / dx[1]) * (ib_basisder1d(n, zero / dx[2]) / dx[2]);
-                    lsg[0] += v * bx;
-                    lsg[1] += v * by;
-                    lsg[2] += v * bz;
-                }
-        const double mag = sqrt(lsg[0] * lsg[0] + lsg[1] * lsg[1] + lsg[2] * lsg[2]);
-        double dist = kZero, xp[3] = {kZero, kZero, kZero};
-        if (mag > kTiny) {
-            dist = (vf - kHalf) / mag;
-#pragma unroll
-            for (int d = 0; d < 3; d++) xp[d] = -dist * (lsg[d] / mag);
-        }
+        double dist, xnd[3];
+        cut_wall(a, i, j, k, xnd, dist);
         const double dxmin = fmin(dx[0], fmin(dx[1], dx[2]));
         const double dnd[3] = {dx[0] / dxmin, dx[1] / dxmin, dx[2] / dxmin};
-        const double xnd[3] = {xp[0] / dxmin, xp[1] / dxmin, xp[2] / dxmin};
         const double cutoff = dxmin * 1e-5;
         const bool doT = !a.conj_ht, doS = !a.spec_in_solid;
         double bD, bP, bT, bV[3], bS[NS];

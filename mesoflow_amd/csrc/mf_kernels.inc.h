@@ -1318,17 +1318,27 @@ __global__ __launch_bounds__(256) void k_fill_list(FillArgs a, const int *list, 
 // update_cutcells (ib_utils.H:271-436), one thread per cut cell of the list;
 // the result goes to cutbuf, the state array is not modified.
 // ---------------------------------------------------------------------------
-MFD double ib_basis1d(int l, double z) {
-    if (l == -1) return kHalf * z * (z - kOne);
-    if (l == 0) return (kOne - z * z);
-    if (l == 1) return kHalf * z * (z + kOne);
-    return 0.0;
-}
-MFD double ib_basisder1d(int l, double z) {
-    if (l == -1) return kHalf * (kTwo * z - kOne);
-    if (l == 0) return -kTwo * z;
-    if (l == 1) return kHalf * (kTwo * z + kOne);
-    return 0.0;
+// the wall point of cut cell (i, j, k) over dxmin, relative to the cell, and the
+// signed distance to it, from the level-set gradient at the centre (:271-300).
+// Of the reference's 27-point quadratic basis only the two neighbours along
+// each axis have a weight there, +-1/(2 dx). Their difference is formed first:
+// it is exactly 0 for equal neighbours, as in the reference's sum of rounded
+// products, where a sum of fused multiply-adds leaves the rounding error of a
+// product, far above kTiny.
+MFD void cut_wall(const CutArgs &a, int i, int j, int k, double *xnd, double &dist) {
+    const View &s = a.s;
+    const double *c = s.p + s.off(i, j, k) + (int64_t)VFRAC * s.ns;
+    const double g[3] = {(c[1] - c[-1]) * (kHalf / a.dx[0]), (c[s.js] - c[-s.js]) * (kHalf / a.dx[1]),
+                         (c[s.ks] - c[-s.ks]) * (kHalf / a.dx[2])};
+    const double dxmin = fmin(a.dx[0], fmin(a.dx[1], a.dx[2]));
+    const double mag = sqrt(g[0] * g[0] + g[1] * g[1] + g[2] * g[2]);
+    dist = kZero;
+    xnd[0] = xnd[1] = xnd[2] = kZero;
+    if (mag > kTiny) {
+        dist = (c[0] - kHalf) / mag;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) xnd[d] = -dist * (g[d] / mag) / dxmin;
+    }
 }
 
 template <class P>
@@ -1341,31 +1351,10 @@ MFD void cutcell_values(const Tab &T, const CutArgs &a, int i, int j, int k, dou
     const double vf = out[VFRAC];
     if (!(vf > kZero && vf < kOne)) return;
     const double *dx = a.dx;
-    // level-set gradient from the 27-point quadratic basis at the centre:
-    // only the (+-1,0,0)-type terms are non-zero, in loop order n,m,l
-    double lsg[3] = {0.0, 0.0, 0.0};
-    const double zero = 0.0;
-    for (int n = -1; n <= 1; n++)
-        for (int m = -1; m <= 1; m++)
-            for (int l = -1; l <= 1; l++) {
-                double v = s(i + l, j + m, k + n, VFRAC);
-                double bx = ib_basisder1d(l, zero / dx[0]) / dx[0] * ib_basis1d(m, zero / dx[1]) * ib_basis1d(n, zero / dx[2]);
-                double by = ib_basis1d(l, zero / dx[0]) * (ib_basisder1d(m, zero / dx[1]) / dx[1]) * ib_basis1d(n, zero / dx[2]);
-                double bz = ib_basis1d(l, zero / dx[0]) * ib_basis1d(m, zero / dx[1]) * (ib_basisder1d(n, zero / dx[2]) / dx[2]);
-                lsg[0] += v * bx;
-                lsg[1] += v * by;
-                lsg[2] += v * bz;
-            }
-    double mag = sqrt(lsg[0] * lsg[0] + lsg[1] * lsg[1] + lsg[2] * lsg[2]);
-    double dist = kZero, xp[3] = {kZero, kZero, kZero};
-    if (mag > kTiny) {
-        dist = (vf - kHalf) / mag;
-#pragma unroll
-        for (int d = 0; d < 3; d++) xp[d] = -dist * (lsg[d] / mag);
-    }
+    double dist, xnd[3];
+    cut_wall(a, i, j, k, xnd, dist);
     const double dxmin = fmin(dx[0], fmin(dx[1], dx[2]));
     const double dnd[3] = {dx[0] / dxmin, dx[1] / dxmin, dx[2] / dxmin};
-    const double xnd[3] = {xp[0] / dxmin, xp[1] / dxmin, xp[2] / dxmin};
     const double cutoff = dxmin * 1e-5;
     // Dirichlet (u = 0) IDW of the velocities, :98-152
     if (fabs(dist) < cutoff) {
@@ -1457,31 +1446,10 @@ MFD int xcd_chunk(int b, int G) {
 MFD void cut_geom_cell(const CutArgs &a, int i, int j, int k, double *g, unsigned *mb) {
     const View &s = a.s;
     const double *dx = a.dx;
-    const double vf = s(i, j, k, VFRAC);
-    double lsg[3] = {0.0, 0.0, 0.0};
-    const double zero = 0.0;
-    for (int n = -1; n <= 1; n++)
-        for (int m = -1; m <= 1; m++)
-            for (int l = -1; l <= 1; l++) {
-                double v = s(i + l, j + m, k + n, VFRAC);
-                double bx = ib_basisder1d(l, zero / dx[0]) / dx[0] * ib_basis1d(m, zero / dx[1]) * ib_basis1d(n, zero / dx[2]);
-                double by = ib_basis1d(l, zero / dx[0]) * (ib_basisder1d(m, zero / dx[1]) / dx[1]) * ib_basis1d(n, zero / dx[2]);
-                double bz = ib_basis1d(l, zero / dx[0]) * ib_basis1d(m, zero / dx[1]) * (ib_basisder1d(n, zero / dx[2]) / dx[2]);
-                lsg[0] += v * bx;
-                lsg[1] += v * by;
-                lsg[2] += v * bz;
-            }
-    double mag = sqrt(lsg[0] * lsg[0] + lsg[1] * lsg[1] + lsg[2] * lsg[2]);
-    double dist = kZero, xp[3] = {kZero, kZero, kZero};
-    if (mag > kTiny) {
-        dist = (vf - kHalf) / mag;
-#pragma unroll
-        for (int d = 0; d < 3; d++) xp[d] = -dist * (lsg[d] / mag);
-    }
     const double dxmin = fmin(dx[0], fmin(dx[1], dx[2]));
     const double dnd[3] = {dx[0] / dxmin, dx[1] / dxmin, dx[2] / dxmin};
-#pragma unroll
-    for (int d = 0; d < 3; ++d) g[d] = xp[d] / dxmin;
+    double dist;
+    cut_wall(a, i, j, k, g, dist);
     g[3] = dist;
     mb[0] = mb[1] = mb[2] = mb[3] = 0u;
     double swv = 0.0, sws = 0.0;
@@ -1704,19 +1672,8 @@ __global__ __launch_bounds__(256) void k_cutcells_box(CutArgs a) {
         const int64_t q = q0 + list[e];
         int i, j, k;
         cell(q, i, j, k);
-        const double *c = s.p + s.off(i, j, k) + (int64_t)VFRAC * s.ns;
-        // the level-set gradient of cut_geom_cell: of the 27-point quadratic
-        // basis only the two neighbours along each axis have a weight
-        const double g0 = (c[1] - c[-1]) * (kHalf / a.dx[0]), g1 = (c[s.js] - c[-s.js]) * (kHalf / a.dx[1]),
-                     g2 = (c[s.ks] - c[-s.ks]) * (kHalf / a.dx[2]);
-        const double mag = sqrt(g0 * g0 + g1 * g1 + g2 * g2);
-        double dist = kZero, xnd[3] = {kZero, kZero, kZero};
-        if (mag > kTiny) {
-            dist = (c[0] - kHalf) / mag;
-            xnd[0] = -dist * (g0 / mag) / dxmin;
-            xnd[1] = -dist * (g1 / mag) / dxmin;
-            xnd[2] = -dist * (g2 / mag) / dxmin;
-        }
+        double dist, xnd[3];
+        cut_wall(a, i, j, k, xnd, dist);
         const bool vel0 = fabs(dist) < dxmin * 1e-5;
         CutSums<NS> o = {};
         for (int r = lane; r < 25; r += kCutLanes) {
