@@ -501,7 +501,7 @@ struct Rev {
     // adjoint of the output (lb, NV) into the adjoint of the input S3 in place.
     // -----------------------------------------------------------------------
     MFD static void post_cell(const Tab &T, double *S, double dt, int clip) {
-        if (P::kHasChemistry) chemistry_rk3<P>(T, S, dt);
+        if (P::kHasChemistry) chemistry_rk3<P, kRatesPerStage>(T, S, dt, nullptr);
         if (S[VFRAC] == kOne) {
             double u[NC], p[NCV];
 #pragma unroll
@@ -522,7 +522,7 @@ struct Rev {
         double S[NV];
 #pragma unroll
         for (int n = 0; n < NV; ++n) S[n] = S3[n];
-        if (P::kHasChemistry) chemistry_rk3<P>(T, S, dt);
+        if (P::kHasChemistry) chemistry_rk3<P, kRatesPerStage>(T, S, dt, nullptr);
         // S: after chemistry (input of the primitive update)
         const bool prim = S[VFRAC] == kOne;
         double u[NC], p[NCV];

@@ -184,6 +184,7 @@ struct PShockTubeN2 {
     static constexpr bool kGammaIgnoresP = true;  // gamma does not depend on the pressure
     static constexpr bool kHasBgGas = false;
     template <class C> MFD static void spec_source(const Tab &, const C &, double *src) { src[0] = kZero; }
+    static constexpr int kRates = 0;  // temperature-only rate constants of the source, at most
     MFD static void rate_constants(const Tab &, double, double *) {}
     template <class C> MFD static void spec_source_k(const Tab &T, const double *, const C &cell, double *src) {
         spec_source(T, cell, src);
@@ -277,6 +278,7 @@ struct PCatalystCylinder : PMixture<4, 3> {
         src[2] += reactrate;
     }
     // a constant rate: nothing depends on temperature
+    static constexpr int kRates = 0;
     MFD static void rate_constants(const Tab &, double, double *) {}
     template <class C> MFD static void spec_source_k(const Tab &T, const double *, const C &cell, double *src) {
         spec_source(T, cell, src);
@@ -352,7 +354,18 @@ struct PPorous : PMixture<NSv, NSv - 1> {
 #pragma unroll
         for (int s = 0; s < NS; ++s) wdot[s] = kZero;
         double Tm = cell(TEMP);
-        for (int r = 0; r < T.nreact; ++r) add_reaction(T, r, exp(T.log_A[r] - T.Ea[r] / (T.R_univ * Tm)), cell, wdot);
+        for (int r = 0; r < T.nreact; ++r) add_reaction(T, r, rate_constant(T, r, Tm), cell, wdot);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) src[s] = kZero + wdot[s];
+    }
+    static constexpr int kRates = MF_MAX_REACTIONS;
+    MFD static double rate_constant(const Tab &T, int r, double Tm) { return exp(T.log_A[r] - T.Ea[r] / (T.R_univ * Tm)); }
+    // the source from rate constants k[r * stride] (the same values as spec_source)
+    template <class C> MFD static void spec_source_at(const Tab &T, const double *k, int stride, const C &cell, double *src) {
+        double wdot[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) wdot[s] = kZero;
+        for (int r = 0; r < T.nreact; ++r) add_reaction(T, r, k[r * stride], cell, wdot);
 #pragma unroll
         for (int s = 0; s < NS; ++s) src[s] = kZero + wdot[s];
     }
@@ -362,7 +375,7 @@ struct PPorous : PMixture<NSv, NSv - 1> {
 #pragma unroll
         for (int r = 0; r < MF_MAX_REACTIONS; ++r) {
             k[r] = kZero;
-            if (r < T.nreact) k[r] = exp(T.log_A[r] - T.Ea[r] / (T.R_univ * Tm));
+            if (r < T.nreact) k[r] = rate_constant(T, r, Tm);
         }
     }
     template <class C> MFD static void spec_source_k(const Tab &T, const double *k, const C &cell, double *src) {
@@ -487,6 +500,7 @@ struct PRef {
 #pragma unroll
         for (int s = 0; s < NS; ++s) src[s] = out[FLO + s];
     }
+    static constexpr int kRates = 0;
     MFD static void rate_constants(const Tab &, double, double *) {}
     template <class C> MFD static void spec_source_k(const Tab &T, const double *, const C &cell, double *src) {
         spec_source(T, cell, src);

@@ -713,17 +713,18 @@ struct ChemCell {
     MFD double operator()(int n) const { return n >= FLO ? sp[n - FLO] : S[n]; }
 };
 
-template <class P>
-MFD void chemistry_rk3(const Tab &T, double *S, double dt) {
+// where the rate constants of the plugin's species source come from: formed at
+// every stage, or once (the temperature does not change over the stages), in
+// registers k[r] or in a column of LDS k[r * kPostBlock]
+enum RateForm { kRatesPerStage, kRatesInRegisters, kRatesInLds };
+constexpr int kPostBlock = 256;  // threads of a block of the kernels below, at most
+template <class P, RateForm FORM>
+MFD void chemistry_rk3(const Tab &T, double *S, double dt, const double *rates) {
     constexpr int NS = P::NS;
     if (!P::kHasChemistry) return;
     double S0[NS], F[3][NS], st[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) S0[s] = S[FLO + s];
-    // the temperature does not change over the stages: the rate constants once,
-    // where each stage's source would evaluate the same exponentials
-    double rates[MF_MAX_REACTIONS];
-    P::rate_constants(T, S[TEMP], rates);
     const double a10 = 1.0, a20 = 0.25, a21 = 0.25;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -735,7 +736,9 @@ MFD void chemistry_rk3(const Tab &T, double *S, double dt) {
             st[s] = v;
         }
         double src[NS];
-        P::spec_source_k(T, rates, ChemCell<NS>{S, st}, src);
+        if constexpr (FORM == kRatesInRegisters) P::spec_source_k(T, rates, ChemCell<NS>{S, st}, src);
+        else if constexpr (FORM == kRatesInLds) P::spec_source_at(T, rates, kPostBlock, ChemCell<NS>{S, st}, src);
+        else P::spec_source(T, ChemCell<NS>{S, st}, src);
 #pragma unroll
         for (int s = 0; s < NS; ++s) F[k][s] = 0.0 + src[s];
     }
@@ -747,6 +750,31 @@ MFD void chemistry_rk3(const Tab &T, double *S, double dt) {
         v += (dt * w1) * F[1][s];
         v += (dt * w2) * F[2][s];
         S[FLO + s] = v;
+    }
+}
+// one exponential per reaction and cell instead of three. In LDS (16 KiB a
+// block) the reactions stay a loop; in registers they are unrolled, which took
+// the kernels of 5 species from two waves per SIMD to one (k_post 242 -> 312
+// registers: 1.68 -> 2.61 ms at 256^3; with an exponential per stage 1.70).
+// Those of 10 species hold one wave in either form and are faster with the
+// reactions unrolled (634 us against 718 at 96^3 with 8 reactions; 735 with an
+// exponential per stage).
+template <class P>
+constexpr RateForm kRateForm = P::kRates == 0 ? kRatesPerStage : (P::NS <= 5 ? kRatesInLds : kRatesInRegisters);
+// doubles of the rate columns of a block
+template <class P>
+constexpr int kRateCols = kRateForm<P> == kRatesInLds ? P::kRates * kPostBlock : 1;
+template <class P>
+MFD void chemistry_rk3_rates(const Tab &T, double *S, double dt, double *column) {
+    if constexpr (kRateForm<P> == kRatesInLds) {
+        for (int r = 0; r < T.nreact; ++r) column[r * kPostBlock] = P::rate_constant(T, r, S[TEMP]);
+        chemistry_rk3<P, kRatesInLds>(T, S, dt, column);
+    } else if constexpr (kRateForm<P> == kRatesInRegisters) {
+        double k[MF_MAX_REACTIONS];
+        P::rate_constants(T, S[TEMP], k);
+        chemistry_rk3<P, kRatesInRegisters>(T, S, dt, k);
+    } else {
+        chemistry_rk3<P, kRatesPerStage>(T, S, dt, nullptr);
     }
 }
 
@@ -929,9 +957,10 @@ __global__ __launch_bounds__(256) void k_residual(ResArgs r, Work w) {
 // Advance_chemistry_implicit, update_primitive_vars, clip_neg_speciesconc,
 // compute_residual_norms and EstTimeStep partials, point by point.
 template <class P, bool CHEM>
-__global__ __launch_bounds__(256) void k_post(ResArgs r, Work w) {
+__global__ __launch_bounds__(kPostBlock) void k_post(ResArgs r, Work w) {
     using N = Num<P>;
     constexpr int NS = P::NS, NV = N::NV;
+    __shared__ double rates[CHEM ? kRateCols<P> : 1];
     const StageArgs &a = r.st;
     if (step_skipped(a.ts)) return;
     const Tab &T = *a.tab;
@@ -966,7 +995,7 @@ __global__ __launch_bounds__(256) void k_post(ResArgs r, Work w) {
             if (CHEM) {
 #pragma unroll
                 for (int n = DENS; n < NV; ++n) So_p[n - DENS] = S[n];
-                chemistry_rk3<P>(T, S, dt);
+                chemistry_rk3_rates<P>(T, S, dt, rates + threadIdx.x);
             }
             // update_primitive_vars (mflo_evolve.cpp:129-160)
             if (S[VFRAC] == kOne) {
@@ -1028,9 +1057,10 @@ __global__ __launch_bounds__(256) void k_post(ResArgs r, Work w) {
 // partials, on one box view in place (the per-box form of
 // Advance_chemistry_implicit, update_primitive_vars, clip_neg_speciesconc)
 template <class P>
-__global__ __launch_bounds__(256) void k_box_post(BoxPostArgs a) {
+__global__ __launch_bounds__(kPostBlock) void k_box_post(BoxPostArgs a) {
     using N = Num<P>;
     constexpr int NS = P::NS, NV = N::NV;
+    __shared__ double rates[kRateCols<P>];
     const Tab &T = *a.tab;
     const int64_t nc = (int64_t)a.e[0] * a.e[1] * a.e[2];
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < nc; q += (int64_t)gridDim.x * blockDim.x) {
@@ -1041,7 +1071,7 @@ __global__ __launch_bounds__(256) void k_box_post(BoxPostArgs a) {
         double S[NV];
 #pragma unroll
         for (int n = 0; n < NV; ++n) S[n] = a.s(i, j, k, n);
-        if (a.chem) chemistry_rk3<P>(T, S, a.dt);
+        if (a.chem) chemistry_rk3_rates<P>(T, S, a.dt, rates + threadIdx.x);
         if (a.prims) {
             if (S[VFRAC] == kOne) {
                 double u[N::NC], p[NCV];
@@ -1071,8 +1101,9 @@ __global__ __launch_bounds__(256) void k_box_post(BoxPostArgs a) {
 // list (a level of a hierarchy, whose primitive update waits for the end of
 // the coarse step): st.src -> dst (may alias), dt of st.ts
 template <class P>
-__global__ __launch_bounds__(256) void k_chem_tiles(ResArgs r, Work w) {
+__global__ __launch_bounds__(kPostBlock) void k_chem_tiles(ResArgs r, Work w) {
     constexpr int NV = Num<P>::NV;
+    __shared__ double rates[kRateCols<P>];
     const StageArgs &a = r.st;
     if (step_skipped(a.ts)) return;
     const Tab &T = *a.tab;
@@ -1094,7 +1125,7 @@ __global__ __launch_bounds__(256) void k_chem_tiles(ResArgs r, Work w) {
             double S[NV];
 #pragma unroll
             for (int n = 0; n < NV; ++n) S[n] = sp[(int64_t)n * a.src.ns];
-            chemistry_rk3<P>(T, S, dt);
+            chemistry_rk3_rates<P>(T, S, dt, rates + threadIdx.x);
 #pragma unroll
             for (int n = 0; n < NV; ++n) dp[(int64_t)n * r.dst.ns] = S[n];
         }
