@@ -1346,8 +1346,8 @@ __global__ __launch_bounds__(256) void k_fill_list(FillArgs a, const int *list, 
 }
 
 // ---------------------------------------------------------------------------
-// update_cutcells (ib_utils.H:271-436), one thread per cut cell of the list;
-// the result goes to cutbuf, the state array is not modified.
+// update_cutcells (ib_utils.H:271-436) of the cut cells of a list; the result
+// goes to cutbuf, the state array is not modified.
 // ---------------------------------------------------------------------------
 // the wall point of cut cell (i, j, k) over dxmin, relative to the cell, and the
 // signed distance to it, from the level-set gradient at the centre (:271-300).
@@ -1528,48 +1528,54 @@ __global__ __launch_bounds__(128) void k_cut_geom_sub(CutArgs a, double *geom, u
     for (int w = 0; w < 4; ++w) mask[(int64_t)w * a.ncut + q] = mb[w];
 }
 
-// The IDW sums of one cut cell over its fluid neighbours, by 8 lanes: a lane
-// takes the rows r = lane, lane + 8, .. of the 25 rows (m, n) of five cells, so
-// that neighbours next to each other in memory are read one after the other
-// and a cell's 125 positions are 20 steps long instead of 125; the lanes' sums
-// are then exchanged. One thread a cell walked its neighbours serially: 84 us
-// for the 35 thousand cut cells of a 64^3 reactor, whatever their number.
+// The IDW sums of one cut cell over its fluid neighbours
 template <int NS>
 struct CutSums {
     double su0, su1, su2, swv, sp, sT, sR, swn, sS[NS];
 };
+// neighbour (l, m, n) at c, with one reciprocal per weight, multiplied into each
+// value (the reference divides every value by the squared distance)
+template <int NS>
+MFD void cut_add(const CutArgs &a, const double *c, int l, int m, int n, const double *dnd, const double *xnd, bool vel0,
+                 CutSums<NS> &o) {
+    const int64_t ns = a.s.ns;
+    const bool doT = !a.conj_ht, doS = !a.spec_in_solid;
+    const double a0 = l * dnd[0], a1 = m * dnd[1], a2 = n * dnd[2];
+    if (!vel0 && !(l == 0 && m == 0 && n == 0)) {
+        const double iw = div_pos(1.0, a0 * a0 + a1 * a1 + a2 * a2 + kTiny2);
+        o.su0 += c[(int64_t)VELX * ns] * iw;
+        o.su1 += c[(int64_t)VELY * ns] * iw;
+        o.su2 += c[(int64_t)VELZ * ns] * iw;
+        o.swv += iw;
+    }
+    const double y0 = a0 - xnd[0], y1 = a1 - xnd[1], y2 = a2 - xnd[2];
+    const double iw = div_pos(1.0, y0 * y0 + y1 * y1 + y2 * y2 + kTiny2);
+    o.sp += c[(int64_t)PRES * ns] * iw;
+    if (doT) o.sT += c[(int64_t)TEMP * ns] * iw;
+    o.sR += c[(int64_t)DENS * ns] * iw;
+    if (doS) {
+#pragma unroll
+        for (int q = 0; q < NS; ++q) o.sS[q] += c[(int64_t)(FLO + q) * ns] * iw;
+    }
+    o.swn += iw;
+}
+// By 8 lanes, a lane takes the rows r = lane, lane + 8, .. of the 25 rows (m, n)
+// of five cells, so that neighbours next to each other in memory are read one
+// after the other and a cell's 125 positions are 20 steps long instead of 125;
+// the lanes' sums are then exchanged.
 template <int NS>
 MFD void cut_row(const CutArgs &a, const double *c0, int m, int n, unsigned bits, const double *dnd, const double *xnd,
                  bool vel0, CutSums<NS> &o) {
-    const int64_t ns = a.s.ns;
-    const bool doT = !a.conj_ht, doS = !a.spec_in_solid;
-    const double a1 = m * dnd[1], a2 = n * dnd[2], y1 = a1 - xnd[1], y2 = a2 - xnd[2];
     while (bits) {
-        const int l = __ffs(bits) - 3;
+        const int l = __builtin_ctz(bits) - 2;
         bits &= bits - 1;
-        const double *c = c0 + l;
-        const double a0 = l * dnd[0], y0 = a0 - xnd[0];
-        // one reciprocal per weight, multiplied into each value (the
-        // reference divides every value by the squared distance)
-        if (!vel0 && !(l == 0 && m == 0 && n == 0)) {
-            const double iw = div_pos(1.0, a0 * a0 + a1 * a1 + a2 * a2 + kTiny2);
-            o.su0 += c[(int64_t)VELX * ns] * iw;
-            o.su1 += c[(int64_t)VELY * ns] * iw;
-            o.su2 += c[(int64_t)VELZ * ns] * iw;
-            o.swv += iw;
-        }
-        const double iw = div_pos(1.0, y0 * y0 + y1 * y1 + y2 * y2 + kTiny2);
-        o.sp += c[(int64_t)PRES * ns] * iw;
-        if (doT) o.sT += c[(int64_t)TEMP * ns] * iw;
-        o.sR += c[(int64_t)DENS * ns] * iw;
-        if (doS) {
-#pragma unroll
-            for (int q = 0; q < NS; ++q) o.sS[q] += c[(int64_t)(FLO + q) * ns] * iw;
-        }
-        o.swn += iw;
+        cut_add<NS>(a, c0 + l, l, m, n, dnd, xnd, vel0, o);
     }
 }
 constexpr int kCutLanes = 8;
+// lists of at least this many cells take one lane a cell: both forms take the
+// same time there (between the measured 499 and 928 thousand, see k_cutcells)
+constexpr int kCutOneLane = 600000;
 template <int NS>
 __device__ __forceinline__ void cut_exchange(CutSums<NS> &o) {
     auto red = [](double &v) {
@@ -1581,7 +1587,8 @@ __device__ __forceinline__ void cut_exchange(CutSums<NS> &o) {
 #pragma unroll
     for (int q = 0; q < NS; ++q) red(o.sS[q]);
 }
-// the updated components of cut cell (i, j, k) from its sums
+// the updated components of cut cell (i, j, k) from its sums; out holds the
+// cell's values on entry
 template <class P>
 MFD void cut_finish(const Tab &T, const CutArgs &a, int i, int j, int k, double dist, bool vel0, const CutSums<P::NS> &o,
                     double *out) {
@@ -1590,8 +1597,6 @@ MFD void cut_finish(const Tab &T, const CutArgs &a, int i, int j, int k, double 
     const View &s = a.s;
     const bool doT = !a.conj_ht, doS = !a.spec_in_solid;
     const double dxmin = fmin(a.dx[0], fmin(a.dx[1], a.dx[2]));
-#pragma unroll
-    for (int n = 0; n < NV; ++n) out[n] = s(i, j, k, n);
     // Dirichlet (u = 0) IDW of the velocities, :98-152
     if (vel0) {
         out[VELX] = 0.0; out[VELY] = 0.0; out[VELZ] = 0.0;
@@ -1631,14 +1636,21 @@ MFD void cut_finish(const Tab &T, const CutArgs &a, int i, int j, int k, double 
     for (int c = 0; c < NCV; ++c) out[c] = u[c];
 }
 
-// update_cutcells of the level's cut-cell list (ib_utils.H:271-436), 8 lanes
-// per cut cell, with the static geometry and fluid-neighbour mask of k_cut_geom
-template <class P>
-__global__ __launch_bounds__(256) void k_cutcells(CutArgs a) {
-    constexpr int NS = P::NS, NV = Num<P>::NV;
+// update_cutcells of the level's cut-cell list (ib_utils.H:271-436) with the
+// static geometry and fluid-neighbour mask of k_cut_geom, LANES lanes per cut
+// cell. With 8 a short list still fills the chip and no thread walks its 125
+// neighbours alone; with 1 the lanes of a wave are mostly x-neighbours, whose
+// loads, and the stores of the results, share cache lines. Bound by the latency
+// of the neighbour reads on short lists, by their traffic on long ones. Sphere
+// packs of 5 species, us by 8 lanes / by 1: 38 thousand cells 40 / 83, 273
+// thousand 242 / 329, 499 thousand 471 / 493, 928 thousand 871 / 801, 2.1 million
+// 1973 / 1684.
+template <class P, int LANES>
+__global__ __launch_bounds__(LANES == 1 ? 128 : 256) void k_cutcells(CutArgs a) {
+    constexpr int NS = P::NS, NV = Num<P>::NV, BLOCK = LANES == 1 ? 128 : 256;
     if (step_skipped(a.ts)) return;
-    const int lane = threadIdx.x & (kCutLanes - 1);
-    const int q = xcd_chunk(blockIdx.x, gridDim.x) * (256 / kCutLanes) + threadIdx.x / kCutLanes;
+    const int lane = threadIdx.x % LANES;
+    const int q = xcd_chunk(blockIdx.x, gridDim.x) * (BLOCK / LANES) + threadIdx.x / LANES;
     if (q >= a.ncut) return;
     const View &s = a.s;
     const int i = a.list[q], j = a.list[a.ncut + q], k = a.list[2 * a.ncut + q];
@@ -1648,16 +1660,34 @@ __global__ __launch_bounds__(256) void k_cutcells(CutArgs a) {
     const double dist = a.geom[(int64_t)3 * a.ncut + q];
     const bool vel0 = fabs(dist) < dxmin * 1e-5;
     CutSums<NS> o = {};
-    for (int r = lane; r < 25; r += kCutLanes) {
-        const int nb = r * 5, w = nb >> 5, sh = nb & 31;
-        unsigned bits = a.mask[(int64_t)w * a.ncut + q] >> sh;
-        if (sh > 27) bits |= a.mask[(int64_t)(w + 1) * a.ncut + q] << (32 - sh);
-        const int m = r % 5 - 2, n = r / 5 - 2;
-        cut_row<NS>(a, s.p + s.off(i, j + m, k + n), m, n, bits & 31u, dnd, xnd, vel0, o);
-    }
-    cut_exchange<NS>(o);
-    if (lane != 0) return;
     double out[NV];
+    auto load = [&] {
+#pragma unroll
+        for (int n = 0; n < NV; ++n) out[n] = s(i, j, k, n);
+    };
+    if constexpr (LANES == 1) {
+        load();
+        for (int w = 0; w < 4; ++w) {
+            unsigned bits = a.mask[(int64_t)w * a.ncut + q];
+            while (bits) {
+                const int nb = w * 32 + __builtin_ctz(bits);
+                bits &= bits - 1;
+                const int l = nb % 5 - 2, m = (nb / 5) % 5 - 2, n = nb / 25 - 2;
+                cut_add<NS>(a, s.p + s.off(i + l, j + m, k + n), l, m, n, dnd, xnd, vel0, o);
+            }
+        }
+    } else {
+        for (int r = lane; r < 25; r += LANES) {
+            const int nb = r * 5, w = nb >> 5, sh = nb & 31;
+            unsigned bits = a.mask[(int64_t)w * a.ncut + q] >> sh;
+            if (sh > 27) bits |= a.mask[(int64_t)(w + 1) * a.ncut + q] << (32 - sh);
+            const int m = r % 5 - 2, n = r / 5 - 2;
+            cut_row<NS>(a, s.p + s.off(i, j + m, k + n), m, n, bits & 31u, dnd, xnd, vel0, o);
+        }
+        cut_exchange<NS>(o);
+        if (lane != 0) return;
+        load();
+    }
     cut_finish<P>(*a.tab, a, i, j, k, dist, vel0, o, out);
 #pragma unroll
     for (int n = 0; n < NV; ++n) a.cutbuf[(int64_t)n * a.ncut + q] = out[n];
@@ -1719,6 +1749,8 @@ __global__ __launch_bounds__(256) void k_cutcells_box(CutArgs a) {
         cut_exchange<NS>(o);
         if (lane == 0) {
             double out[NV];
+#pragma unroll
+            for (int n = 0; n < NV; ++n) out[n] = s(i, j, k, n);
             cut_finish<P>(*a.tab, a, i, j, k, dist, vel0, o, out);
 #pragma unroll
             for (int n = 0; n < NV; ++n) a.tmp[(int64_t)n * ncell + q] = out[n];
@@ -1862,10 +1894,16 @@ struct Launch {
     }
     static void cut(const CutArgs &a, hipStream_t st) {
         if (a.ncut <= 0) return;
+        if (a.ncut >= kCutOneLane) {
+            int g = (a.ncut + 127) / 128;
+            g = (g + 7) & ~7;
+            hipLaunchKernelGGL((k_cutcells<P, 1>), dim3(g), dim3(128), 0, st, a);
+            return;
+        }
         const int per = 256 / kCutLanes;
         int g = (a.ncut + per - 1) / per;
         if (g >= 8) g = (g + 7) & ~7;
-        hipLaunchKernelGGL(k_cutcells<P>, dim3(g), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((k_cutcells<P, kCutLanes>), dim3(g), dim3(256), 0, st, a);
     }
     static void cut_geom(const CutArgs &a, double *geom, unsigned *mask, hipStream_t st) {
         if (a.ncut <= 0) return;
