@@ -2068,7 +2068,6 @@ int level_autotune(Level *L) {
     r.old = L->view[0];
     r.dst = L->view[1];
     r.do_ns = c->prm.do_ns;
-    r.partials = L->partials;
     // the fastest of three rounds of three launches (after one untimed): a
     // single round let run-to-run noise pick between near-equal candidates
     auto time_it = [&](auto &&launch) -> double {
@@ -2107,15 +2106,22 @@ int level_autotune(Level *L) {
                 // primitives, norms): it is timed with the residual, reading B
                 // and writing C so that the state in A stays as it was
                 ResArgs rp = r;
-                rp.partials = L->partials;  // rebuild_tiles grows (frees) it with the tile count
+                rp.partials = L->partials;  // of this candidate's tiles: rebuild_tiles grows (frees) it with their number
                 rp.st.src = L->view[1];
                 rp.dst = L->view[2];
                 rp.do_chem = c->prm.do_chemistry;
                 rp.clip = c->prm.clip_species;
                 rp.track_res = c->prm.track_residual_norms;
+                // a pass that would write another buffer than the level's, or past
+                // its end, is not launched: the call returns an error instead
                 auto post = [&] {
-                    c->ks->post(rp, level_work(L, kCellClass), grid_for(L->ntiles[kCellClass], L->max_grid), 256,
-                                c->stream);
+                    const Work w = level_work(L, kCellClass);
+                    const int grid = grid_for(L->ntiles[kCellClass], L->max_grid);
+                    if (rp.partials != L->partials || (size_t)(w.t0 + grid) * (c->nv + 2) > L->partials_cap) {
+                        st = MF_ERR_BAD_ARG;
+                        return;
+                    }
+                    c->ks->post(rp, w, grid, 256, c->stream);
                 };
                 if (!lds) ms = time_it([&] {
                     for (int d = 0; d < 3; ++d) launch_faces(L, a, d, MF_MODE_BATCHED);
@@ -2127,10 +2133,12 @@ int level_autotune(Level *L) {
                     post();
                 });
             }
+            if (st) break;
             if (ms < best) { best = ms; bi[0] = cand[0]; bi[1] = cand[1]; bi[2] = cand[2]; }
         }
         for (int d = 0; d < 3; ++d) L->tsh[cls][d] = bi[d];
-        if (st == MF_OK) st = rebuild_tiles(L);
+        const int rs = rebuild_tiles(L);
+        if (st == MF_OK) st = rs;
     }
     hipEventDestroy(e0);
     hipEventDestroy(e1);

@@ -124,7 +124,8 @@ def test_porous_tiny_boxes():
 def test_autotune_when_a_candidate_has_more_tiles():
     """64 boxes of 16x16x2: 8 cell tiles a box with the default shape 64,2,2 and
     16 with the candidate 64,1,4, so the buffer of the tiles' partial sums grows
-    between two candidates; the post-step pass then writes the new buffer"""
+    between two candidates; the call returns an error (and launches nothing)
+    where the timed post-step pass would not write the new buffer"""
     from mesoflow_amd import runtime
     c = cases.porous_reactor(n_cell=(32, 32, 32), nspec=5, nreact=2, geometry="spheres", porosity=0.6, rmin=3, rmax=5,
                              order_hyp=5, seed=13, max_grid_size=(16, 16, 2))
