@@ -525,6 +525,10 @@ int mf_util_copy(void *ctx, double *dst, const double *src, int64_t n);
  * receives how many quotients equal the IEEE division, differ by one ulp, or
  * by more. */
 int mf_util_div_check(void *ctx, int64_t n, int lo_exp, int hi_exp, int64_t *counts);
+/* The same for the division of the WENO5 increments (at most two ulps off):
+ * counts[4] receives how many quotients equal the IEEE division, differ by one
+ * ulp, by two, or by more. */
+int mf_util_div2_check(void *ctx, int64_t n, int lo_exp, int hi_exp, int64_t *counts);
 
 #ifdef __cplusplus
 }

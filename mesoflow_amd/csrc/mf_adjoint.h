@@ -14,10 +14,10 @@
 namespace mfd {
 
 // ---------------------------------------------------------------------------
-// WENO5-JS (single-division form of Num::weno_plus): gradient w.r.t. s0..s4
-// times gbar, added to sb; returns the reconstructed value (Num::weno_plus up
-// to rounding: one reciprocal of the weight sum instead of a division).
-// weno_minus(s1..s5) == weno_plus(s5,s4,s3,s2,s1).
+// WENO5-JS, the left-biased value s[2] + up of Num::weno_pair in the cell
+// values: gradient w.r.t. s0..s4 times gbar, added to sb; returns the
+// reconstructed value (equal to rounding). The right-biased value of s1..s5 is
+// the left-biased one of s5, s4, s3, s2, s1.
 // ---------------------------------------------------------------------------
 MFD double weno_plus_rev(const double *s, double gbar, double *sb) {
     const double eps = 1e-6;
@@ -54,7 +54,7 @@ MFD double weno_plus_rev(const double *s, double gbar, double *sb) {
     sb[4] += t0b + q0b - v0b;
     return val;
 }
-// gradient of weno_minus(m[0..4]) (m = s1..s5) times gbar, added to mb;
+// gradient of the right-biased value of m[0..4] (m = s1..s5) times gbar, added to mb;
 // returns the reconstructed value
 MFD double weno_minus_rev(const double *m, double gbar, double *mb) {
     const double r[5] = {m[4], m[3], m[2], m[1], m[0]};

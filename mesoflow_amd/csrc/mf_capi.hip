@@ -2161,11 +2161,18 @@ int mf_util_copy(void *ctx, double *dst, const double *src, int64_t n) {
     return MF_OK;
 }
 
-// div_pos against the IEEE division over n seeded operand pairs: numerators
-// of either sign with exponents in [-40, 40], positive denominators with
-// exponents in [lo_exp, hi_exp]; counts[0] equal, [1] one ulp apart, [2] more
-__global__ void k_div_check(int64_t n, int lo_exp, int hi_exp, unsigned long long *counts) {
-    unsigned long long c0 = 0, c1 = 0, c2 = 0;
+}  // extern "C"
+
+namespace {
+// the device divisions against the IEEE division over n seeded operand pairs:
+// numerators of either sign with exponents in [-40, 40], positive denominators
+// with exponents in [lo_exp, hi_exp]; counts[d] quotients d < NCOUNT - 1 ulps
+// apart, the last count more
+template <int NCOUNT, class Div>
+__device__ void div_check(int64_t n, int lo_exp, int hi_exp, unsigned long long *counts, Div div) {
+    unsigned long long cnt[NCOUNT];
+#pragma unroll
+    for (int m = 0; m < NCOUNT; ++m) cnt[m] = 0;
     for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
         // splitmix64 of the index
         uint64_t z = (uint64_t)q * 0x9E3779B97F4A7C15ull + 0x632BE59BD9B4E019ull;
@@ -2181,31 +2188,47 @@ __global__ void k_div_check(int64_t n, int lo_exp, int hi_exp, unsigned long lon
         const int e1 = (int)(r3 % 81) - 40, e2 = lo_exp + (int)(r4 % (uint64_t)(hi_exp - lo_exp + 1));
         const double num = ((r3 >> 32) & 1 ? -1.0 : 1.0) * ldexp(m1, e1);
         const double den = ldexp(m2, e2);
-        const double a = num / den, b = div_pos(num, den);
-        const int64_t ia = __double_as_longlong(a), ib = __double_as_longlong(b);
+        const int64_t ia = __double_as_longlong(num / den), ib = __double_as_longlong(div(num, den));
         const int64_t d = ia > ib ? ia - ib : ib - ia;
-        if (d == 0) ++c0;
-        else if (d == 1) ++c1;
-        else ++c2;
+#pragma unroll
+        for (int m = 0; m < NCOUNT; ++m)
+            if (m == NCOUNT - 1 ? d >= m : d == m) ++cnt[m];
     }
-    atomicAdd(counts + 0, c0);
-    atomicAdd(counts + 1, c1);
-    atomicAdd(counts + 2, c2);
+#pragma unroll
+    for (int m = 0; m < NCOUNT; ++m) atomicAdd(counts + m, cnt[m]);
 }
-
-int mf_util_div_check(void *ctx, int64_t n, int lo_exp, int hi_exp, int64_t *counts) {
+__global__ void k_div_check(int64_t n, int lo_exp, int hi_exp, unsigned long long *counts) {
+    div_check<3>(n, lo_exp, hi_exp, counts, [](double a, double b) { return div_pos(a, b); });
+}
+__global__ void k_div2_check(int64_t n, int lo_exp, int hi_exp, unsigned long long *counts) {
+    div_check<4>(n, lo_exp, hi_exp, counts, [](double a, double b) { return div_pos_2ulp(a, b); });
+}
+int run_div_check(void *ctx, int64_t n, int lo_exp, int hi_exp, int64_t *counts, int ncount,
+                  void (*kernel)(int64_t, int, int, unsigned long long *)) {
     Ctx *c = (Ctx *)ctx;
     if (!c || n < 0 || !counts || lo_exp > hi_exp || lo_exp < -900 || hi_exp > 900) return MF_ERR_BAD_ARG;
     unsigned long long *d = nullptr;
-    HIPCHK(hipMalloc(&d, 3 * sizeof(unsigned long long)));
-    HIPCHK(hipMemsetAsync(d, 0, 3 * sizeof(unsigned long long), c->stream));
-    hipLaunchKernelGGL(k_div_check, dim3(2048), dim3(256), 0, c->stream, n, lo_exp, hi_exp, d);
-    unsigned long long h[3];
-    HIPCHK(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+    const size_t bytes = (size_t)ncount * sizeof(unsigned long long);
+    HIPCHK(hipMalloc(&d, bytes));
+    HIPCHK(hipMemsetAsync(d, 0, bytes, c->stream));
+    hipLaunchKernelGGL(kernel, dim3(2048), dim3(256), 0, c->stream, n, lo_exp, hi_exp, d);
+    unsigned long long h[4] = {0, 0, 0, 0};
+    HIPCHK(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     hipFree(d);
-    for (int q = 0; q < 3; ++q) counts[q] = (int64_t)h[q];
+    for (int q = 0; q < ncount; ++q) counts[q] = (int64_t)h[q];
     return MF_OK;
+}
+}  // namespace
+
+extern "C" {
+
+int mf_util_div_check(void *ctx, int64_t n, int lo_exp, int hi_exp, int64_t *counts) {
+    return run_div_check(ctx, n, lo_exp, hi_exp, counts, 3, k_div_check);
+}
+
+int mf_util_div2_check(void *ctx, int64_t n, int lo_exp, int hi_exp, int64_t *counts) {
+    return run_div_check(ctx, n, lo_exp, hi_exp, counts, 4, k_div2_check);
 }
 
 int mf_adjoint_forward(void *level, int nsteps, int ncheck, int spec, double *J_out) {

@@ -97,8 +97,8 @@ struct CellArr {
 MFD double std_max(double a, double b) { return (a < b) ? b : a; }
 MFD double std_min(double a, double b) { return (b < a) ? b : a; }
 
-// n / d for a positive d far inside the normal range (WENO weight sums,
-// densities, heat capacities, sums of concentrations or of transport
+// n / d for a positive d far inside the normal range (the adjoint's WENO weight
+// sums, densities, heat capacities, sums of concentrations or of transport
 // coefficients plus 1e-30): v_rcp_f64 estimate refined by
 // two Newton-Raphson steps r += r (1 - d r) and one residual correction
 // q += r (n - d q) -- the steps of the full division without the exponent
@@ -117,11 +117,12 @@ MFD double div_pos(double n, double d) {
 #endif
 }
 
-// n / d within about one ulp, for the same denominators: the v_rcp_f64 estimate
+// n / d within two ulps, for the same denominators: the v_rcp_f64 estimate
 // (relative error below 2^-23) refined once to third order, r (1 + e + e^2)
-// with e = 1 - d r, without div_pos's residual correction. For corrections that
-// are added to a larger value (the WENO5 increments).
-MFD double div_pos_1ulp(double n, double d) {
+// with e = 1 - d r (remainder e^3 < 2^-69, one rounding of 2^-53), and the
+// rounding of the product, without div_pos's residual correction. For
+// corrections that are added to a larger value (the WENO5 increments).
+MFD double div_pos_2ulp(double n, double d) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const double r = __builtin_amdgcn_rcp(d);
     double e = fma(-d, r, 1.0);
@@ -644,67 +645,14 @@ struct Num {
         // (adding p_half*0 to the others is exact)
         fh[RHOU + D] += p_half;
     }
-    // WENO5-JS half of flux_schemes.H:400-421 (left-biased value at the face
-    // between s2 and s3) and :423-444 (right-biased value), eps = 1e-6, p = 2,
-    // linear weights (0.1, 0.6, 0.3). With q_k = (eps + beta_k)^2 the nonlinear
-    // weights alpha_k = d_k / q_k are normalised with one division:
-    //   sum_k alpha_k v_k / sum_k alpha_k
-    //     = (v2 q1 q0 + 6 v1 q2 q0 + 3 v0 q2 q1) / (q1 q0 + 6 q2 q0 + 3 q2 q1)
-    // (the reference forms 1/q_k and 1/sum alpha; the value is the same to
-    // rounding). Building with MF_WENO_REFERENCE_DIVISIONS restores the
-    // reference's four divisions.
-    MFD static double weno_combine(double b2, double b1, double b0, double v2, double v1, double v0) {
-        const double eps = 1e-6;
-#ifdef MF_WENO_REFERENCE_DIVISIONS
-        b2 = 1.0 / ((eps + b2) * (eps + b2));
-        b1 = 1.0 / ((eps + b1) * (eps + b1));
-        b0 = 1.0 / ((eps + b0) * (eps + b0));
-        double a2 = b2, a1 = 6.0 * b1, a0 = 3.0 * b0;
-        double alpha1 = 1.0 / (a2 + a1 + a0);
-        return (1.0 / 6.0) * alpha1 * (a2 * v2 + a1 * v1 + a0 * v0);
-#else
-        const double q2 = (eps + b2) * (eps + b2);
-        const double q1 = (eps + b1) * (eps + b1);
-        const double q0 = (eps + b0) * (eps + b0);
-        const double w2 = q1 * q0, w1 = 6.0 * (q2 * q0), w0 = 3.0 * (q2 * q1);
-        return div_pos(w2 * v2 + w1 * v1 + w0 * v0, 6.0 * (w2 + w1 + w0));
-#endif
-    }
-    MFD static double weno_plus(double s0, double s1, double s2, double s3, double s4) {
-        double t = s0 - 2.0 * s1 + s2;
-        double q = s0 - 4.0 * s1 + 3.0 * s2;
-        const double b2 = (13.0 / 12.0) * (t * t) + 0.25 * (q * q);
-        t = s1 - 2.0 * s2 + s3;
-        const double b1 = (13.0 / 12.0) * (t * t) + 0.25 * (s1 - s3) * (s1 - s3);
-        t = s2 - 2.0 * s3 + s4;
-        q = 3.0 * s2 - 4.0 * s3 + s4;
-        const double b0 = (13.0 / 12.0) * (t * t) + 0.25 * (q * q);
-        const double v2 = 2.0 * s0 - 7.0 * s1 + 11.0 * s2;
-        const double v1 = -s1 + 5.0 * s2 + 2.0 * s3;
-        const double v0 = 2.0 * s2 + 5.0 * s3 - s4;
-        return weno_combine(b2, b1, b0, v2, v1, v0);
-    }
-    MFD static double weno_minus(double s1, double s2, double s3, double s4, double s5) {
-        double t = s5 - 2.0 * s4 + s3;
-        double q = s5 - 4.0 * s4 + 3.0 * s3;
-        const double b2 = (13.0 / 12.0) * (t * t) + 0.25 * (q * q);
-        t = s4 - 2.0 * s3 + s2;
-        const double b1 = (13.0 / 12.0) * (t * t) + 0.25 * (s4 - s2) * (s4 - s2);
-        t = s3 - 2.0 * s2 + s1;
-        q = 3.0 * s3 - 4.0 * s2 + s1;
-        const double b0 = (13.0 / 12.0) * (t * t) + 0.25 * (q * q);
-        const double v2 = 11.0 * s3 - 7.0 * s4 + 2.0 * s5;
-        const double v1 = -s4 + 5.0 * s3 + 2.0 * s2;
-        const double v0 = 2.0 * s3 + 5.0 * s2 - s1;
-        return weno_combine(b2, b1, b0, v2, v1, v0);
-    }
-    // Both WENO5-JS values at the face between s[2] and s[3] as increments,
-    // left-biased s[2] + up and right-biased s[3] - um, in the differences
-    // d_k = s[k+1] - s[k] and t_k = d_{k+1} - d_k: the same smoothness
-    // indicators, weights and candidates as weno_plus / weno_minus (times 4 and
-    // over 6), with the second differences shared by the two sides. 71 FP64
-    // operations for the pair (112 for weno_plus and weno_minus), and the
-    // increments carry no cancellation of the cell value.
+    // Both WENO5-JS values at the face between s[2] and s[3] (left-biased
+    // flux_schemes.H:400-421, right-biased :423-444; eps = 1e-6, p = 2, linear
+    // weights 0.1, 0.6, 0.3) as increments, left-biased s[2] + up and right-biased
+    // s[3] - um, in the differences d_k = s[k+1] - s[k] and t_k = d_{k+1} - d_k:
+    // the reference's smoothness indicators (times 4), weights and candidates
+    // (less the cell value), with the second differences shared by the two sides.
+    // 71 FP64 operations for the pair (112 for one side at a time in the cell
+    // values), and the increments carry no cancellation of the cell value.
     MFD static void weno_pair(const double *s, double &up, double &um) {
         const double d0 = s[1] - s[0], d1 = s[2] - s[1], d2 = s[3] - s[2], d3 = s[4] - s[3], d4 = s[5] - s[4];
         const double t0 = d1 - d0, t1 = d2 - d1, t2 = d3 - d2, t3 = d4 - d3;
@@ -718,15 +666,26 @@ struct Num {
     static constexpr double k13Thirds = 13.0 / 3.0, kWenoEps4 = 4.0e-6;
     // one side: first-derivative parts q and second-derivative parts c of the
     // outer, middle and inner stencil; differences a0, a1 on the upwind side, a2
-    // across the face, a3 beyond it
+    // across the face, a3 beyond it. With s_k = (eps + beta_k)^2 the nonlinear
+    // weights d_k / s_k are normalised with one division,
+    //   sum_k (d_k / s_k) p_k / sum_k (d_k / s_k)
+    //     = (p2 s1 s0 + 6 p1 s2 s0 + 3 p0 s2 s1) / (s1 s0 + 6 s2 s0 + 3 s2 s1)
+    // (the reference forms 1/s_k and the reciprocal of their sum; the value is
+    // the same to rounding). Building with MF_WENO_REFERENCE_DIVISIONS restores
+    // the reference's four divisions.
     MFD static double weno_increment(double q2, double q1, double q0, double c2, double c1, double c0, double a0, double a1,
                                      double a2, double a3) {
         const double b2 = fma(q2, q2, c2), b1 = fma(q1, q1, c1), b0 = fma(q0, q0, c0);
         const double s2 = b2 * b2, s1 = b1 * b1, s0 = b0 * b0;
-        const double w2 = s1 * s0, w1 = s2 * s0, w0 = s2 * s1;
         const double p2 = fma(5.0 / 6.0, a1, (-1.0 / 3.0) * a0), p1 = fma(2.0, a2, a1), p0 = fma(2.0, a2, -kHalf * a3);
+#ifdef MF_WENO_REFERENCE_DIVISIONS
+        const double w2 = 1.0 / s2, w1 = 1.0 / s1, w0 = 1.0 / s0;
+        return (w0 * p0 + w1 * p1 + w2 * p2) * (1.0 / (3.0 * w0 + 6.0 * w1 + w2));
+#else
+        const double w2 = s1 * s0, w1 = s2 * s0, w0 = s2 * s1;
         const double n = fma(w0, p0, fma(w1, p1, w2 * p2)), d = fma(3.0, w0, fma(6.0, w1, w2));
-        return div_pos_1ulp(n, d);
+        return div_pos_2ulp(n, d);
+#endif
     }
     // LLF flux of one component from its six states u and fluxes f
     // (flux_schemes.H:448-495): (f+ + lam u+)/2 + (f- - lam u-)/2

@@ -101,6 +101,7 @@ SIGNATURES = {
     "mf_hier_read_checkpoint": ([C.c_void_p, C.c_char_p, _P(C.c_char_p)], C.c_int),
     "mf_util_copy": ([C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64], C.c_int),
     "mf_util_div_check": ([C.c_void_p, C.c_int64, C.c_int, C.c_int, C.c_void_p], C.c_int),
+    "mf_util_div2_check": ([C.c_void_p, C.c_int64, C.c_int, C.c_int, C.c_void_p], C.c_int),
 }
 
 

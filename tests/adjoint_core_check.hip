@@ -116,33 +116,88 @@ static double dot(const std::vector<double> &a, const std::vector<double> &b) {
 }
 
 // ---------------------------------------------------------------------------
+// WENO5-JS as in the textbook (and flux_schemes.H:400-444), in extended
+// precision: the left-biased value at the face between s2 and s3
+static long double weno_textbook(long double s0, long double s1, long double s2, long double s3, long double s4) {
+    const long double eps = 1e-6L, c = 13.0L / 12.0L;
+    auto sq = [](long double x) { return x * x; };
+    const long double b2 = c * sq(s0 - 2 * s1 + s2) + 0.25L * sq(s0 - 4 * s1 + 3 * s2);
+    const long double b1 = c * sq(s1 - 2 * s2 + s3) + 0.25L * sq(s1 - s3);
+    const long double b0 = c * sq(s2 - 2 * s3 + s4) + 0.25L * sq(3 * s2 - 4 * s3 + s4);
+    const long double a2 = 0.1L / sq(eps + b2), a1 = 0.6L / sq(eps + b1), a0 = 0.3L / sq(eps + b0);
+    const long double v2 = (2 * s0 - 7 * s1 + 11 * s2) / 6, v1 = (-s1 + 5 * s2 + 2 * s3) / 6, v0 = (2 * s2 + 5 * s3 - s4) / 6;
+    return (a2 * v2 + a1 * v1 + a0 * v0) / (a2 + a1 + a0);
+}
+// the values the kernels form, on both sides of the face
+static double pair_left(const double *s) {
+    double up, um;
+    Num<P>::weno_pair(s, up, um);
+    return s[2] + up;
+}
+static double pair_right(const double *s) {
+    double up, um;
+    Num<P>::weno_pair(s, up, um);
+    return s[3] - um;
+}
+static void check_weno_pair() {
+    // uniform, linear, smooth, jumps at every position, one spike, random; scaled
+    // from 1e-6 to 1e8 (densities to total energies), with and without an offset.
+    // The differences are exact to one ulp of the cell values, weights and
+    // candidates follow with relative errors of a few ulps: 128 ulps of the
+    // largest cell value in all
+    double worst = 0.0;
+    int n = 0;
+    for (int shape = 0; shape < 14; ++shape)
+        for (int e = -6; e <= 8; ++e)
+            for (int off = 0; off < 2; ++off) {
+                double s[6], big = 0.0;
+                for (int q = 0; q < 6; ++q) {
+                    double x = 0.0;
+                    if (shape == 1) x = 0.1 * q;
+                    else if (shape == 2) x = sin(0.4 * q);
+                    else if (shape >= 3 && shape <= 7) x = q >= shape - 2 ? 1.0 : 0.1;
+                    else if (shape >= 8 && shape <= 12) x = q == shape - 8 ? 1.0 : 0.0;
+                    else if (shape == 13) x = urand(-1, 1);
+                    s[q] = (x + off * 3.0) * pow(10.0, e);
+                    big = fmax(big, fabs(s[q]));
+                }
+                const double l = (double)fabsl(pair_left(s) - weno_textbook(s[0], s[1], s[2], s[3], s[4]));
+                const double r = (double)fabsl(pair_right(s) - weno_textbook(s[5], s[4], s[3], s[2], s[1]));
+                const double tol = 128 * 1.2e-16 * big;
+                if (big > 0) worst = fmax(worst, fmax(l, r) / big);
+                if (!(l <= tol && r <= tol)) {
+                    printf("weno_pair shape %d scale 1e%d offset %d: off by %.3e %.3e FAIL\n", shape, e, off, l, r);
+                    ++failures;
+                }
+                ++n;
+            }
+    printf("weno_pair against the textbook form: %d stencils, worst %.2e of the largest cell value\n", n, worst);
+}
 static void check_weno() {
+    check_weno_pair();
     for (int trial = 0; trial < 4; ++trial) {
-        double s[5], v[5], w = urand(-2, 2);
-        for (int q = 0; q < 5; ++q) { s[q] = urand(-1, 1) * (trial + 1); v[q] = urand(-1, 1); }
-        if (trial == 3) for (int q = 0; q < 5; ++q) s[q] = 0.3 + 0.01 * q + 1e-4 * urand(-1, 1);  // smooth data
+        // s[0..5]: the left-biased value reads s[0..4], the right-biased one s[1..5]
+        double s[6], v[6], w = urand(-2, 2);
+        for (int q = 0; q < 6; ++q) { s[q] = urand(-1, 1) * (trial + 1); v[q] = urand(-1, 1); }
+        if (trial == 3) for (int q = 0; q < 6; ++q) s[q] = 0.3 + 0.01 * q + 1e-4 * urand(-1, 1);  // smooth data
         double g[5] = {0, 0, 0, 0, 0}, gm[5] = {0, 0, 0, 0, 0};
         const double vp = weno_plus_rev(s, w, g);
-        const double vm = weno_minus_rev(s, w, gm);
-        // the reverse passes return the forward reconstructions (to rounding)
+        const double vm = weno_minus_rev(s + 1, w, gm);
+        // the reverse passes return the forward reconstructions of the kernels (to rounding)
         {
-            const double fp = Num<P>::weno_plus(s[0], s[1], s[2], s[3], s[4]);
-            const double fm = Num<P>::weno_minus(s[0], s[1], s[2], s[3], s[4]);
             char nm[64];
             snprintf(nm, sizeof nm, "weno_plus value trial %d", trial);
-            report(nm, vp, fp, 1e-14);
+            report(nm, vp, pair_left(s), 1e-14);
             snprintf(nm, sizeof nm, "weno_minus value trial %d", trial);
-            report(nm, vm, fm, 1e-14);
+            report(nm, vm, pair_right(s), 1e-14);
         }
         double ad = 0, adm = 0;
-        for (int q = 0; q < 5; ++q) { ad += g[q] * v[q]; adm += gm[q] * v[q]; }
+        for (int q = 0; q < 5; ++q) { ad += g[q] * v[q]; adm += gm[q] * v[q + 1]; }
         const double h = 1e-6;
-        double sp[5], sm[5];
-        for (int q = 0; q < 5; ++q) { sp[q] = s[q] + h * v[q]; sm[q] = s[q] - h * v[q]; }
-        const double fd = w * (Num<P>::weno_plus(sp[0], sp[1], sp[2], sp[3], sp[4]) -
-                               Num<P>::weno_plus(sm[0], sm[1], sm[2], sm[3], sm[4])) / (2 * h);
-        const double fdm = w * (Num<P>::weno_minus(sp[0], sp[1], sp[2], sp[3], sp[4]) -
-                                Num<P>::weno_minus(sm[0], sm[1], sm[2], sm[3], sm[4])) / (2 * h);
+        double sp[6], sm[6];
+        for (int q = 0; q < 6; ++q) { sp[q] = s[q] + h * v[q]; sm[q] = s[q] - h * v[q]; }
+        const double fd = w * (pair_left(sp) - pair_left(sm)) / (2 * h);
+        const double fdm = w * (pair_right(sp) - pair_right(sm)) / (2 * h);
         char nm[64];
         snprintf(nm, sizeof nm, "weno_plus trial %d", trial);
         report(nm, ad, fd, 1e-6);
