@@ -687,6 +687,16 @@ struct Num {
         return div_pos_2ulp(n, d);
 #endif
     }
+    // component c of geteulerflux (consprim_funcs.H:68-80) for direction D from the
+    // component u itself, the normal velocity and the pressure. rho v_a is the
+    // momentum; the reference divides and multiplies by rho again, which differs
+    // in the last bit.
+    template <int D>
+    MFD static double weno_flux(int c, double u, double vn, double p) {
+        if (c == RHOU + D) return fma(u, vn, p);
+        if (c == RHOE) return (u + p) * vn;
+        return u * vn;
+    }
     // LLF flux of one component from its six states u and fluxes f
     // (flux_schemes.H:448-495): (f+ + lam u+)/2 + (f- - lam u-)/2
     MFD static double weno_llf(const double *u, const double *f, double lam) {

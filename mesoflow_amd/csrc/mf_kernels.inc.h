@@ -247,13 +247,13 @@ MFD void face_flux(const Tab &T, const Acc &acc, const StageArgs &a, int i, int 
                 load(pR, ur);
                 lam = N::template max_eigenvalue<D>(T, ul, ur);
             }
-            double pr[6][5];  // rho, vx, vy, vz, p of the six stencil cells
+            double vn[6], pr[6];  // normal velocity and pressure of the six stencil cells
 #pragma unroll
             for (int q = 0; q < 6; ++q) {
-                double u[NC];
+                double u[NC], v[3];
                 load(cp[q], u);
-                pr[q][0] = u[RHO];
-                N::euler_prims(T, u, pr[q][1], pr[q][2], pr[q][3], pr[q][4]);
+                N::euler_prims(T, u, v[0], v[1], v[2], pr[q]);
+                vn[q] = v[D];
             }
 #pragma unroll 1
             for (int c = 0; c < NC; ++c) {
@@ -262,14 +262,7 @@ MFD void face_flux(const Tab &T, const Acc &acc, const StageArgs &a, int i, int 
 #pragma unroll
                 for (int q = 0; q < 6; ++q) {
                     uc[q] = cp[q](comp);
-                    const double vn = pr[q][1 + D];
-                    if (c == RHO) fc[q] = pr[q][0] * vn;
-                    else if (c >= RHOU && c <= RHOW) {
-                        const double va = (c == RHOU) ? pr[q][1] : ((c == RHOV) ? pr[q][2] : pr[q][3]);
-                        const double m = pr[q][0] * va;
-                        fc[q] = (c - RHOU == D) ? (m * va + pr[q][4]) : (m * vn);
-                    } else if (c == RHOE) fc[q] = (uc[q] + pr[q][4]) * vn;
-                    else fc[q] = uc[q] * vn;
+                    fc[q] = N::template weno_flux<D>(c, uc[q], vn[q], pr[q]);
                 }
                 fput(c, adv(c, N::weno_llf(uc, fc, lam)));
             }
@@ -576,11 +569,7 @@ __global__ __launch_bounds__(512, MF_FACE_MIN_WAVES) void k_faces_lds(StageArgs 
                     for (int q = 0; q < 6; ++q) {
                         const double *rq = rs[q];
                         uc[q] = rq[c];
-                        const double vn = rq[FVN];
-                        // geteulerflux with rho v_a taken as the momentum itself
-                        if (c == RHOU + D) fc[q] = fma(uc[q], vn, rq[FP]);
-                        else if (c == RHOE) fc[q] = (uc[q] + rq[FP]) * vn;
-                        else fc[q] = uc[q] * vn;
+                        fc[q] = N::template weno_flux<D>(c, uc[q], rq[FVN], rq[FP]);
                     }
                     hc[c] = N::weno_llf(uc, fc, lam);
                 }
@@ -680,7 +669,7 @@ __global__ __launch_bounds__(512, MF_FACE_MIN_WAVES) void k_faces_lds(StageArgs 
                     for (int q = 0; q < 6; ++q) {
                         const double *rq = rs[q];
                         uc[q] = rq[c];
-                        fc[q] = uc[q] * rq[FVN];
+                        fc[q] = uc[q] * rq[FVN];  // weno_flux of a species
                     }
                     hc[c] = T.advect_flag[c - NCV] * N::weno_llf(uc, fc, lam);
                 }
