@@ -677,13 +677,16 @@ struct Num {
                                      double a2, double a3) {
         const double b2 = fma(q2, q2, c2), b1 = fma(q1, q1, c1), b0 = fma(q0, q0, c0);
         const double s2 = b2 * b2, s1 = b1 * b1, s0 = b0 * b0;
-        const double p2 = fma(5.0 / 6.0, a1, (-1.0 / 3.0) * a0), p1 = fma(2.0, a2, a1), p0 = fma(2.0, a2, -kHalf * a3);
 #ifdef MF_WENO_REFERENCE_DIVISIONS
         const double w2 = 1.0 / s2, w1 = 1.0 / s1, w0 = 1.0 / s0;
-        return (w0 * p0 + w1 * p1 + w2 * p2) * (1.0 / (3.0 * w0 + 6.0 * w1 + w2));
 #else
         const double w2 = s1 * s0, w1 = s2 * s0, w0 = s2 * s1;
+#endif
+        const double p2 = fma(5.0 / 6.0, a1, (-1.0 / 3.0) * a0), p1 = fma(2.0, a2, a1), p0 = fma(2.0, a2, -kHalf * a3);
         const double n = fma(w0, p0, fma(w1, p1, w2 * p2)), d = fma(3.0, w0, fma(6.0, w1, w2));
+#ifdef MF_WENO_REFERENCE_DIVISIONS
+        return n * (1.0 / d);
+#else
         return div_pos_2ulp(n, d);
 #endif
     }
