@@ -1,9 +1,10 @@
 // mf_device.h -- device numerics of the RHS path for gfx950 (FP64 throughout).
 //
 // Each function states the reference lines whose arithmetic it reproduces.
-// Operation order follows the reference expression by expression (the build
-// turns FP contraction off), so that results agree with the reference's CPU
-// build to rounding. pow(x,2) is written x*x and pow(x,-1) as 1/x.
+// Operation order follows the reference expression by expression where nothing
+// else is said, so that results agree with the reference's CPU build to rounding
+// (the build lets a*b+c become one fused operation). pow(x,2) is written x*x and
+// pow(x,-1) as 1/x.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

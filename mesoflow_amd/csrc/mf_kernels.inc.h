@@ -1275,10 +1275,10 @@ MFD void ghost_cell(int64_t q, int64_t nzs, int64_t nys, int PX, int PY, int nx,
     }
 }
 
-// the ghost cells of a padded level array in one launch: bound by launches at
-// small sizes, by the reads of the domain shell at large ones (12 us a fill at
-// 64^3 and 108 us at 256^3 with 17 components, timed between events that cost 6;
-// four launches, one per number of outside directions, took 27 and 162)
+// the ghost cells of a padded level array in one launch: bound by the launch at
+// small sizes, by the reads of the domain shell at large ones (4.6 us a fill for
+// 32x4x4 cells, 111 us at 256^3 with 17 components; four launches, one per number
+// of outside directions, took 19 and 159)
 template <class P>
 __global__ __launch_bounds__(256) void k_fill(FillArgs a) {
     if (step_skipped(a.ts)) return;
@@ -1686,7 +1686,7 @@ __global__ __launch_bounds__(LANES == 1 ? 128 : 256) void k_cutcells(CutArgs a) 
 // set. A block collects the cut cells among its 256 cells and gives each to 8
 // lanes, with the geometry computed on the way: about one cell in eight of a
 // packed bed is cut, and one thread a cell left the others of its wave waiting
-// for 250 serial neighbour reads (123 us for a 32^3 box).
+// for 250 serial neighbour reads (124 us for a 32^3 box, 38 this way).
 template <class P>
 __global__ __launch_bounds__(256) void k_cutcells_box(CutArgs a) {
     constexpr int NS = P::NS, NV = Num<P>::NV;
